@@ -25,6 +25,7 @@
 #include "kernels.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace nnchip
 {
@@ -314,6 +315,675 @@ namespace nnchip
 						mr.m.y[t * mr.m.y_stride + mr.r + r] = v;
 					else
 						p.part[(static_cast<size_t>(split) * nt + t) * p.rows + row0 + r] = v;
+				}
+			}
+		}
+
+		// ---- 17 vectors and more: gemv_batch_kernel and gemv_tile_kernel ----
+		//
+		// X is split into bf16 hi + lo once per call (gemv_stage_x_kernel) and
+		// the products go the other way round: A = X (16 vectors x 32 columns),
+		// B = the rows' weights, so D holds vectors 4 (l / 16) + i of row
+		// l % 16: a row's scale is one value per lane and Y's rows are
+		// consecutive lanes. Batches of 512 vectors ran 16 at a time through
+		// gemv_kernel before, the weights read 32 times over.
+
+		// 64 bytes of each of 16 weight rows per wavefront load (a "piece", 16
+		// bytes per lane: row l % 16, bytes 16 (l / 16) ..): this many 32-column
+		// blocks.
+		template <int F>
+		constexpr int kPieceBlocks = F == kGemvBf16 ? 1 : (F == kGemvQ8_0 ? 2 : 4);
+
+		__device__ __forceinline__ u32x2 swap32(uint32_t a, uint32_t b)
+		{
+			const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+			return u32x2{r[0], r[1]};
+		}
+		__device__ __forceinline__ u32x2 swap16(uint32_t a, uint32_t b)
+		{
+			const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+			return u32x2{r[0], r[1]};
+		}
+
+		// The B operands (16 rows x 32 columns each) of a piece's blocks. The
+		// columns that lane group g = l / 16 holds of a block (and so must hold
+		// of X): BF16 8 g .. 8 g + 7; Q8_0 16 (g % 2) + 8 (g / 2) .. + 7; Q4_S
+		// 4 g .. 4 g + 3 and 16 + 4 g .. + 3.
+		template <int F>
+		__device__ __forceinline__ void batch_operands(const u32x4& w, bf16x8 (&b)[kPieceBlocks<F>])
+		{
+			if constexpr (F == kGemvBf16)
+				b[0] = as_bf16x8(w);
+			else if constexpr (F == kGemvQ8_0)
+			{
+				// The piece holds block 0 in lane groups 0, 1 and block 1 in 2, 3:
+				// exchanging halves gives each block to all four groups.
+				const u32x2 d0 = swap32(w[0], w[2]), d1 = swap32(w[1], w[3]);
+				b[0] = q8_to_bf16x8(d0.x, d1.x);
+				b[1] = q8_to_bf16x8(d0.y, d1.y);
+			}
+			else
+			{
+				// Lane group g holds block g's four dwords; block j wants dword g
+				// in group g: a 4 x 4 transpose.
+				const u32x2 s02 = swap32(w[0], w[2]), s13 = swap32(w[1], w[3]);
+				const u32x2 b01 = swap16(s02.x, s13.x), b23 = swap16(s02.y, s13.y);
+				b[0] = q4_to_bf16x8(b01.x);
+				b[1] = q4_to_bf16x8(b01.y);
+				b[2] = q4_to_bf16x8(b23.x);
+				b[3] = q4_to_bf16x8(b23.y);
+			}
+		}
+
+		// The sum of a block's 32 x on every lane of a vector (lane l: vector
+		// l % 16, x[0..3] columns 4 g .. and x[4..7] columns 16 + 4 g .., g =
+		// l / 16), added as the reference does (reference nn_ops.cpp:1305-1316
+		// under its -ffast-math build: l_j = (x_j + x_8+j) + (x_16+j + x_24+j),
+		// then ((l0 + l4) + (l1 + l5)) + ((l2 + l6) + (l3 + l7))).
+		__device__ __forceinline__ float batch_block_sum(const float (&x)[8])
+		{
+			float u[4];
+#pragma unroll
+			for (int j = 0; j < 4; ++j)
+				u[j] = add_with_other_row(add_with_other_half(x[j]) + add_with_other_half(x[4 + j]));
+			return (u[0] + u[1]) + (u[2] + u[3]);
+		}
+
+		// The first of a lane's columns in a block, and where its second four are.
+		template <int F>
+		__device__ __forceinline__ int x_first_col(int grp)
+		{
+			return F == kGemvBf16 ? 8 * grp : (F == kGemvQ8_0 ? 16 * (grp & 1) + 8 * (grp >> 1) : 4 * grp);
+		}
+		template <int F>
+		constexpr int kXSecond = F == kGemvQ4S ? 16 : 4;
+
+		// X^T of a 32-column block and a tile of 16 vectors as the A operand (lane
+		// l: vector l % 16, its columns of the block), split into bf16 hi + lo,
+		// from the lane's eight values as loaded.
+		__device__ __forceinline__ void x_operands(const u32x4& a, const u32x4& b, bf16x8& hi, bf16x8& lo)
+		{
+			const float4 f = __builtin_bit_cast(float4, a), g = __builtin_bit_cast(float4, b);
+			const float o[8] = {f.x, f.y, f.z, f.w, g.x, g.y, g.z, g.w};
+			split_bf16x8(o, hi, lo);
+		}
+
+		// X of a whole call as operands in memory (p.xs, written by
+		// gemv_stage_x_kernel): per (block, tile of 16 vectors) 1 KB of hi and
+		// 1 KB of lo in lane order, so a wavefront's load is 1 KB of consecutive
+		// addresses, where the vectors themselves lie cols * 4 bytes apart (16
+		// lines per load, for many widths on one L2 channel). For Q4_S then the
+		// block sums as operands of a product over blocks: per (32 blocks,
+		// tile) 1 KB each of hi, mid and lo, the three bf16 that hold a sum's
+		// 24 bits (lane l: vector l % 16, blocks 8 (l / 16) .. + 7).
+		__device__ __forceinline__ u32x4* x_staged(const gemv_params& p, int blk, int tile)
+		{
+			return static_cast<u32x4*>(p.xs) + (static_cast<size_t>(blk) * p.x_tiles + tile) * 128;
+		}
+		__device__ __forceinline__ uint16_t* x_sums(const gemv_params& p, int step, int tile)
+		{
+			const size_t n = static_cast<size_t>(p.cols / 32) * p.x_tiles;
+			return reinterpret_cast<uint16_t*>(static_cast<u32x4*>(p.xs) + n * 128) +
+			       (static_cast<size_t>(step) * p.x_tiles + tile) * 1536;
+		}
+
+		// One wavefront per (block, tile); Q4_S: also the blocks that fill up the
+		// last 32 (sums of zero). Vectors past the last one repeat it.
+		template <int F>
+		__global__ __launch_bounds__(256) void gemv_stage_x_kernel(const gemv_params p)
+		{
+			const int lane = threadIdx.x & 63, item = blockIdx.x * 4 + (threadIdx.x >> 6);
+			const int nb = p.cols / 32, blk = item / p.x_tiles, tile = item % p.x_tiles;
+			if (blk >= (F == kGemvQ4S ? (nb + 31) & ~31 : nb)) return; // the whole wavefront
+			const int t = min(16 * tile + (lane & 15), p.n_batch - 1);
+			const float* x = p.x + static_cast<size_t>(t) * p.x_stride + 32 * min(blk, nb - 1) + x_first_col<F>(lane >> 4);
+			const u32x4 a = *reinterpret_cast<const u32x4*>(x), b = *reinterpret_cast<const u32x4*>(x + kXSecond<F>);
+			if (blk < nb)
+			{
+				bf16x8 hi, lo;
+				x_operands(a, b, hi, lo);
+				u32x4* o = x_staged(p, blk, tile) + lane;
+				o[0] = __builtin_bit_cast(u32x4, hi);
+				o[64] = __builtin_bit_cast(u32x4, lo);
+			}
+			if constexpr (F == kGemvQ4S)
+			{
+				const float4 f = __builtin_bit_cast(float4, a), g = __builtin_bit_cast(float4, b);
+				const float v[8] = {f.x, f.y, f.z, f.w, g.x, g.y, g.z, g.w};
+				float s = batch_block_sum(v);
+				if (blk >= nb)
+					s = 0.0f;
+				else if (p.xsum)
+					s = p.xsum[static_cast<size_t>(t) * p.xsum_stride + blk];
+				if (lane < 16)
+				{
+					uint16_t* o = x_sums(p, blk >> 5, tile) + (lane + 16 * ((blk & 31) >> 3)) * 8 + (blk & 7);
+					const uint32_t h = f32_to_bf16_bits(s);
+					const float r = s - bf16_bits_to_f32(h);
+					const uint32_t m = f32_to_bf16_bits(r);
+					o[0] = static_cast<uint16_t>(h);
+					o[512] = static_cast<uint16_t>(m);
+					o[1024] = static_cast<uint16_t>(f32_to_bf16_bits(r - bf16_bits_to_f32(m)));
+				}
+			}
+		}
+
+		// 16 bytes per lane from byte off + s_off of the buffer to LDS, 1 KB from
+		// dst on in lane order.
+		__device__ __forceinline__ void dma_lds16(__amdgpu_buffer_rsrc_t r, unsigned char* dst, uint32_t off, uint32_t s_off)
+		{
+			typedef __attribute__((address_space(3))) void* lds_ptr;
+			__builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)dst, 16, off, s_off, 0, 0);
+		}
+
+		// 16 rows of each of RT tiles (rows past the last one repeat it; they are
+		// not stored), read through one buffer descriptor per tile. A piece goes
+		// to LDS by LDS-DMA with four lanes on each row's 64 bytes (row l / 4),
+		// and comes back one 16-byte read per lane in the operand's order (row
+		// l % 16): loads in that order straight to registers put 16 rows in each
+		// quarter wavefront, 64 line lookups per KB, and held a CU to 16 bytes
+		// per clock whatever their depth. The 16-byte slots of a row are XORed
+		// with row / 4, so a quarter wavefront's reads fall on distinct banks.
+		// What lies past a row's end or the wavefront's pieces is loaded from an
+		// offset past the descriptor's, which gives zeros without a memory
+		// access, so no load (and no product) is under a branch: the counts of
+		// loads in flight stay exact.
+		constexpr uint32_t kDeadOffset = 0x80000000u;
+		template <int F, int RT>
+		struct batch_rows
+		{
+			__amdgpu_buffer_rsrc_t w[RT], sc[RT];
+			uint32_t off[RT], s_off[RT]; // this lane's row and its 16 bytes of a piece; its scale
+			const uint16_t* bi[RT];
+			int nb;
+			uint32_t row_bytes, lane_bytes;
+			__device__ __forceinline__ batch_rows(const gemv_params& p, int row0)
+			{
+				const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+				nb = p.cols / 32;
+				row_bytes = static_cast<uint32_t>(nb) * (64 / kPieceBlocks<F>);
+				lane_bytes = 16u * ((lane & 3) ^ grp);
+#pragma unroll
+				for (int r = 0; r < RT; ++r)
+				{
+					const int t0 = min(row0 + 16 * r, (p.rows - 1) & ~15), n = min(16, p.rows - t0);
+					const mat_row mr = locate(p, t0);
+					w[r] = __builtin_amdgcn_make_buffer_rsrc(
+						const_cast<char*>(static_cast<const char*>(mr.m.w) + static_cast<size_t>(mr.r) * row_bytes), 0,
+						static_cast<int>(n * row_bytes), 0x00020000);
+					off[r] = static_cast<uint32_t>(min(lane >> 2, n - 1)) * row_bytes + lane_bytes;
+					const uint32_t row = min(col, n - 1);
+					if constexpr (F != kGemvBf16)
+					{
+						sc[r] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(mr.m.scales + static_cast<size_t>(mr.r) * nb),
+						                                          0, n * nb * 2, 0x00020000);
+						s_off[r] = (row * nb + (grp & (kPieceBlocks<F> - 1))) * 2;
+					}
+					bi[r] = F == kGemvQ4S ? mr.m.biases + (static_cast<size_t>(mr.r) + row) * nb : nullptr;
+				}
+			}
+			// Piece i of tile r into 1 KB of LDS if it is one of the caller's
+			// (below end), and the scale of block (l / 16) % kPieceBlocks of it.
+			__device__ __forceinline__ void load(unsigned char* dst, uint32_t& scale, int r, int i, int end) const
+			{
+				const bool live = i < end && 64u * i + lane_bytes < row_bytes;
+				dma_lds16(w[r], dst, live ? off[r] + 64u * i : kDeadOffset, 0);
+				if constexpr (F != kGemvBf16)
+				{
+					const int grp = (threadIdx.x & 63) >> 4;
+					const bool ok = i < end && kPieceBlocks<F> * i + (grp & (kPieceBlocks<F> - 1)) < nb;
+					scale = __builtin_amdgcn_raw_buffer_load_b16(sc[r], ok ? s_off[r] + 2u * kPieceBlocks<F> * i : kDeadOffset, 0, 0);
+				}
+			}
+			// The piece's 16 bytes of row l % 16, quarter l / 16.
+			static __device__ __forceinline__ u32x4 read(const unsigned char* piece)
+			{
+				const int col = threadIdx.x & 15, grp = (threadIdx.x & 63) >> 4;
+				return *reinterpret_cast<const u32x4*>(piece + 64 * col + 16 * (grp ^ (col >> 2)));
+			}
+		};
+
+		// A piece's scales, each on every lane, from load()'s.
+		template <int F>
+		__device__ __forceinline__ void batch_scales(uint32_t scale, float (&s)[4])
+		{
+			const uint32_t x = scale << 16;
+			if constexpr (F == kGemvQ8_0)
+			{
+				const u32x2 v = swap16(x, x); // rows 0 1 0 1
+				s[0] = __uint_as_float(v.x);
+				s[1] = __uint_as_float(v.y);
+			}
+			else if constexpr (F == kGemvQ4S)
+			{
+				const u32x2 h = swap32(x, x); // rows 0 1 0 1, rows 2 3 2 3
+				const u32x2 lo = swap16(h.x, h.x), hi = swap16(h.y, h.y);
+				s[0] = __uint_as_float(lo.x);
+				s[1] = __uint_as_float(lo.y);
+				s[2] = __uint_as_float(hi.x);
+				s[3] = __uint_as_float(hi.y);
+			}
+		}
+
+		// acc += one block's products of a 16-row tile and a 16-vector tile.
+		template <int F>
+		__device__ __forceinline__ void batch_product(f32x4& acc, const bf16x8& xh, const bf16x8& xl, const bf16x8& w, float s)
+		{
+			if constexpr (F == kGemvBf16)
+			{
+				acc = mfma16x16x32(xh, w, acc);
+				acc = mfma16x16x32(xl, w, acc);
+			}
+			else
+			{
+				f32x4 d = mfma16x16x32(xh, w, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+				d = mfma16x16x32(xl, w, d);
+#pragma unroll
+				for (int i = 0; i < 4; ++i) acc[i] = fmaf(s, d[i], acc[i]);
+			}
+		}
+
+		// s_waitcnt vmcnt(n), the other counters not waited on (gfx9 encoding:
+		// vmcnt[3:0], expcnt[6:4] = 7, lgkmcnt[11:8] = 0xf, vmcnt[5:4] at
+		// bits 15:14). Nothing is scheduled across it.
+		template <int N>
+		__device__ __forceinline__ void wait_loads()
+		{
+			static_assert(N < 64, "vmcnt");
+			__builtin_amdgcn_sched_barrier(0);
+			__builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+			__builtin_amdgcn_sched_barrier(0);
+		}
+
+		// Eight biases of a row from block b0 on as a B operand (zero past the
+		// row's end).
+		__device__ __forceinline__ bf16x8 bias_operand(const uint16_t* bi, int b0, int nb)
+		{
+			uint32_t h[8];
+#pragma unroll
+			for (int i = 0; i < 8; ++i)
+			{
+				const uint32_t v = bi[min(b0 + i, nb - 1)];
+				h[i] = b0 + i < nb ? v : 0u;
+			}
+			return as_bf16x8(u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)});
+		}
+
+		constexpr int kBatchWaves = 8;
+		// Pieces in flight per wavefront (their X with them: loads complete in
+		// order, so X fetched any later would wait for every W load before it).
+		template <int F, int RT, int TT>
+		constexpr int kBatchDepth = F == kGemvBf16 ? (TT == 2 ? 4 : 2) : F == kGemvQ8_0 ? (TT == 2 ? 2 : 1) : 1;
+
+		// Y[t][r] for 16 RT rows per work-group and up to 16 TT vectors, W
+		// streamed once. The wavefronts split the columns (contiguous runs of
+		// whole pieces, the same whatever RT and the number of rows, so a row
+		// gets the same bits in any group) and run without a barrier until
+		// their sums meet in LDS, added in wavefront order: no K splits over
+		// work-groups, no partials in memory and no second launch. A = X (16
+		// vectors x 32 columns, bf16 hi + lo), B = the rows' weights, so D holds
+		// vectors 4 (l / 16) + i of row l % 16: a row's scale is one value per
+		// lane, and Y's rows are consecutive lanes. X comes as operands
+		// (gemv_stage_x_kernel).
+		template <int F, int RT, int TT>
+		__global__ __launch_bounds__(64 * kBatchWaves) void gemv_batch_kernel(const gemv_params p)
+		{
+			constexpr int PB = kPieceBlocks<F>, D = kBatchDepth<F, RT, TT>;
+			// Loads of one piece: X's, the weights' and their scales'.
+			constexpr int NL = 2 * PB * TT + RT * (F == kGemvBf16 ? 1 : 2);
+			extern __shared__ __attribute__((aligned(16))) unsigned char s_raw[];
+			const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+			const int grp = lane >> 4;
+			const int nb = p.cols / 32, np = (nb + PB - 1) / PB;
+			const int i_lo = wave * np / kBatchWaves, i_hi = (wave + 1) * np / kBatchWaves;
+			const int row0 = blockIdx.x * 16 * RT;
+			const batch_rows<F, RT> rows(p, row0);
+			unsigned char* const s_w = s_raw + wave * D * RT * 1024; // [D][RT] pieces of this wavefront
+
+			struct piece_t
+			{
+				u32x4 xh[PB][TT], xl[PB][TT];
+				uint32_t scale[RT];
+			} ring[D];
+			const uint32_t xs_block = static_cast<uint32_t>(p.x_tiles) * 2048u;
+			const __amdgpu_buffer_rsrc_t rx =
+				__builtin_amdgcn_make_buffer_rsrc(x_staged(p, min(i_lo * PB, nb - 1), 0), 0, 0x7fffffff, 0x00020000);
+			auto load = [&](piece_t& k, int d, int i) __attribute__((always_inline))
+			{
+#pragma unroll
+				for (int j = 0; j < PB; ++j)
+				{
+					const int b = i * PB + j;
+					const bool live = i < i_hi && b < nb; // uniform
+					const uint32_t o = live ? (b - i_lo * PB) * xs_block + 16u * lane : kDeadOffset;
+#pragma unroll
+					for (int t = 0; t < TT; ++t)
+					{
+						k.xh[j][t] = __builtin_amdgcn_raw_buffer_load_b128(rx, o, 2048 * t, 0);
+						k.xl[j][t] = __builtin_amdgcn_raw_buffer_load_b128(rx, o, 2048 * t + 1024, 0);
+					}
+				}
+#pragma unroll
+				for (int r = 0; r < RT; ++r) rows.load(s_w + (d * RT + r) * 1024, k.scale[r], r, i, i_hi);
+			};
+
+			f32x4 acc[RT][TT];
+#pragma unroll
+			for (int r = 0; r < RT; ++r)
+#pragma unroll
+				for (int t = 0; t < TT; ++t) acc[r][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+#pragma unroll
+			for (int d = 0; d < D; ++d)
+			{
+				load(ring[d], d, i_lo + d);
+				__builtin_amdgcn_sched_barrier(0);
+			}
+			for (int i0 = i_lo; i0 < i_hi; i0 += D)
+			{
+#pragma unroll
+				for (int d = 0; d < D; ++d)
+				{
+					piece_t& k = ring[d];
+					wait_loads<(D - 1) * NL>(); // this piece's have landed
+					bf16x8 wb[RT][PB];
+					float sc[RT][4];
+#pragma unroll
+					for (int r = 0; r < RT; ++r)
+					{
+						batch_operands<F>(rows.read(s_w + (d * RT + r) * 1024), wb[r]);
+						batch_scales<F>(k.scale[r], sc[r]);
+					}
+#pragma unroll
+					for (int j = 0; j < PB; ++j)
+#pragma unroll
+						for (int t = 0; t < TT; ++t)
+#pragma unroll
+							for (int r = 0; r < RT; ++r)
+								batch_product<F>(acc[r][t], as_bf16x8(k.xh[j][t]), as_bf16x8(k.xl[j][t]), wb[r][j], sc[r][j]);
+					// (kept in this order, or the scheduler gathers the loads at
+					// the loop's end and the next piece waits for all of them;
+					// the piece's LDS reads have returned: the products took them)
+					__builtin_amdgcn_sched_barrier(0);
+					load(k, d, i0 + d + D);
+					__builtin_amdgcn_sched_barrier(0);
+				}
+			}
+			wait_loads<0>(); // (zeros on their way to LDS)
+			__syncthreads(); // the sums take the pieces' place
+			f32x4* s_sum = reinterpret_cast<f32x4*>(s_raw); // [wavefront][RT][TT][64]
+			if constexpr (F == kGemvQ4S)
+			{
+				// The bias term, bias . (block sums of x), 32 blocks per product,
+				// the products in turn over the wavefronts.
+				for (int st = wave; st < (nb + 31) / 32; st += kBatchWaves)
+#pragma unroll
+					for (int r = 0; r < RT; ++r)
+					{
+						const bf16x8 b = bias_operand(rows.bi[r], 32 * st + 8 * grp, nb);
+#pragma unroll
+						for (int t = 0; t < TT; ++t)
+						{
+							const u32x4* xs = reinterpret_cast<const u32x4*>(x_sums(p, st, t)) + lane;
+#pragma unroll
+							for (int i = 2; i >= 0; --i) acc[r][t] = mfma16x16x32(as_bf16x8(xs[64 * i]), b, acc[r][t]);
+						}
+					}
+			}
+
+#pragma unroll
+			for (int r = 0; r < RT; ++r)
+#pragma unroll
+				for (int t = 0; t < TT; ++t) s_sum[((wave * RT + r) * TT + t) * 64 + lane] = acc[r][t];
+			__syncthreads();
+			const float* s_f = reinterpret_cast<const float*>(s_raw);
+			for (int i = threadIdx.x; i < RT * TT * 256; i += 64 * kBatchWaves)
+			{
+				const int rl = i & 15, tl = (i >> 4) & 15, tile = i >> 8; // tile = r * TT + t
+				const int row = row0 + 16 * (tile / TT) + rl, tok = 16 * (tile % TT) + tl;
+				const float* f = s_f + tile * 256 + 4 * (rl + 16 * (tl >> 2)) + (tl & 3);
+				float v[kBatchWaves], sum = 0.0f;
+#pragma unroll
+				for (int w = 0; w < kBatchWaves; ++w) v[w] = f[w * RT * TT * 256];
+#pragma unroll
+				for (int w = 0; w < kBatchWaves; ++w) sum = w == 0 ? v[0] : sum + v[w];
+				if (row < p.rows && tok < p.n_batch)
+				{
+					const mat_row mr = locate(p, row);
+					mr.m.y[tok * mr.m.y_stride + mr.r] = sum;
+				}
+			}
+		}
+
+		// ---- many vectors: gemv_tile_kernel ----
+
+		// Y of 16 RT WR rows and 16 TT vectors per work-group: WR groups of 16 RT
+		// rows for each of two groups over the columns, one wavefront each. X's
+		// operands arrive in LDS by LDS-DMA as they lie staged, one block a
+		// slot, in a ring of SLOTS slots per column group, shared by the row
+		// groups; a wavefront's own weights in a ring of NPW pieces. The column
+		// groups' sums meet in LDS at the end. Work-groups of one row tile run
+		// on one XCD, so a weight comes from HBM once and from that XCD's L2 for
+		// the other vectors.
+		template <int F, int RT, int TT, int WR, int SLOTS, int NPW>
+		struct tile_shape
+		{
+			static constexpr int PB = kPieceBlocks<F>;
+			static constexpr int WB = NPW * PB; // blocks of W in flight
+			static constexpr int U = SLOTS > WB ? SLOTS : WB; // blocks per loop pass (a multiple of both)
+			static constexpr int kSlot = TT * 2048;
+			static constexpr int DX = TT * 2 / WR; // X's DMAs per wavefront and block
+			static constexpr int NW = RT * (F == kGemvBf16 ? 1 : 2); // weight and scale loads per piece
+			static constexpr int kLdsX = 2 * SLOTS * kSlot;
+			static constexpr int kLds = kLdsX + 2 * WR * NPW * RT * 1024;
+			static_assert(TT * 2 % WR == 0 && (U == 2 || U == 4 || U == 8) && U % SLOTS == 0 && U % WB == 0, "tile shape");
+			static_assert(WR * RT * TT * 1024 <= kLds, "the sums reuse the rings");
+			// Loads a wavefront may have in flight at the top of block j with X
+			// and W of block j landed: those asked for after both. Block b asks
+			// for X of block b + SLOTS - 1 at its top, and at its end, if it is
+			// a piece's last, for the piece WB blocks on.
+			static constexpr int in_flight(int j)
+			{
+				int n = 0, since = 0; // since the later of the two
+				for (int b = j - 2 * U; b < j; ++b)
+				{
+					n += DX;
+					if (b + SLOTS - 1 == j) since = n;
+					if ((b + 4 * U + 1) % PB == 0)
+					{
+						n += NW;
+						const int first = b + 1 - PB + WB;
+						if (first <= j && j < first + PB) since = n;
+					}
+				}
+				return n - since;
+			}
+		};
+
+		template <int F, int RT, int TT, int WR, int SLOTS, int NPW>
+		__global__ __launch_bounds__(128 * WR) void gemv_tile_kernel(const gemv_params p)
+		{
+			using S = tile_shape<F, RT, TT, WR, SLOTS, NPW>;
+			constexpr int PB = S::PB, U = S::U, WB = S::WB;
+			extern __shared__ __attribute__((aligned(16))) unsigned char s_raw[];
+			const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+			const int col = lane & 15, grp = lane >> 4;
+			const int wr = wave % WR, kg = wave / WR;
+			const int nb = p.cols / 32;
+			const int n_tt = (p.x_tiles + TT - 1) / TT, n_rt = (p.rows + 16 * RT * WR - 1) / (16 * RT * WR);
+			// (row tile, vector tile): the vector tiles of a row tile consecutive on one XCD
+			int rt, tt;
+			{
+				const int xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
+				rt = 8 * (i / n_tt) + xcd;
+				tt = i % n_tt;
+			}
+			if (rt >= n_rt) return; // the whole work-group
+			const int row0 = (rt * WR + wr) * 16 * RT;
+			const batch_rows<F, RT> rows(p, row0);
+
+			// Column group kg takes blocks b_lo .. b_lo + h - 1 (whole pieces),
+			// as far as there are any.
+			const int np = (nb + PB - 1) / PB, h = (np + 1) / 2 * PB;
+			const int b_lo = kg * h, p_hi = min(np, (kg + 1) * (h / PB));
+
+			const uint32_t xs_block = static_cast<uint32_t>(p.x_tiles) * 2048u;
+			const __amdgpu_buffer_rsrc_t rx =
+				__builtin_amdgcn_make_buffer_rsrc(x_staged(p, min(b_lo, nb - 1), 0), 0, 0x7fffffff, 0x00020000);
+			unsigned char* const s_x = s_raw + kg * SLOTS * S::kSlot;
+			unsigned char* const s_w = s_raw + S::kLdsX + wave * NPW * RT * 1024; // [NPW][RT] pieces of this wavefront
+			uint32_t x_off[S::DX]; // DMA u: 1 KB (hi or lo of a tile) to its place [tile][hi, lo] in the slot
+#pragma unroll
+			for (int u = 0; u < S::DX; ++u)
+			{
+				const int e = u * WR + wr;
+				x_off[u] = 2048u * min(tt * TT + e / 2, p.x_tiles - 1) + 1024u * (e & 1) + 16u * lane;
+			}
+			// X of block i of the group into slot i % SLOTS.
+			auto load_x = [&](int i, int slot) __attribute__((always_inline))
+			{
+				const bool live = i < h && b_lo + i < nb; // uniform
+#pragma unroll
+				for (int u = 0; u < S::DX; ++u)
+					dma_lds16(rx, s_x + slot * S::kSlot + 1024 * (u * WR + wr), live ? x_off[u] : kDeadOffset,
+					          live ? i * xs_block : 0u);
+			};
+			uint32_t scale[NPW][RT];
+			f32x4 acc[RT][TT];
+#pragma unroll
+			for (int r = 0; r < RT; ++r)
+#pragma unroll
+				for (int t = 0; t < TT; ++t) acc[r][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+			// The loop's order of loads, begun before its first block.
+#pragma unroll
+			for (int b = -U; b < 0; ++b)
+			{
+				if (b >= 1 - SLOTS) load_x(b + SLOTS - 1, (b + SLOTS - 1) % SLOTS);
+				__builtin_amdgcn_sched_barrier(0);
+				if (b >= -WB && (b + WB + 1) % PB == 0)
+				{
+					const int q = (b + WB) / PB; // the piece's slot, and its number in the group
+#pragma unroll
+					for (int r = 0; r < RT; ++r) rows.load(s_w + (q * RT + r) * 1024, scale[q][r], r, b_lo / PB + q, p_hi);
+				}
+				__builtin_amdgcn_sched_barrier(0);
+			}
+			for (int i0 = 0; i0 < h; i0 += U)
+			{
+				auto block = [&](auto j_tag) __attribute__((always_inline))
+				{
+					constexpr int j = decltype(j_tag)::value, q = (j % WB) / PB;
+					wait_loads<S::in_flight(j)>();
+					// Everyone's X of block j, and everyone is done with the slot
+					// reused next (its reads have returned: the products took
+					// them). The bare barrier: __syncthreads() would wait for
+					// the loads in flight.
+					__builtin_amdgcn_s_barrier();
+					__builtin_amdgcn_sched_barrier(0);
+					load_x(i0 + j + SLOTS - 1, (j + SLOTS - 1) % SLOTS);
+					__builtin_amdgcn_sched_barrier(0);
+					u32x4 wv[RT];
+#pragma unroll
+					for (int r = 0; r < RT; ++r) wv[r] = rows.read(s_w + (q * RT + r) * 1024);
+					const u32x4* xs = reinterpret_cast<const u32x4*>(s_x + (j % SLOTS) * S::kSlot) + lane;
+					bf16x8 xh[TT], xl[TT];
+#pragma unroll
+					for (int t = 0; t < TT; ++t)
+					{
+						xh[t] = as_bf16x8(xs[t * 128]);
+						xl[t] = as_bf16x8(xs[t * 128 + 64]);
+					}
+					__builtin_amdgcn_sched_barrier(0);
+					bf16x8 wb[RT];
+					float sb[RT];
+#pragma unroll
+					for (int r = 0; r < RT; ++r)
+					{
+						bf16x8 all[PB];
+						float sc[4];
+						batch_operands<F>(wv[r], all);
+						batch_scales<F>(scale[q][r], sc);
+						wb[r] = all[j % PB];
+						sb[r] = sc[j % PB];
+					}
+#pragma unroll
+					for (int t = 0; t < TT; ++t)
+#pragma unroll
+						for (int r = 0; r < RT; ++r) batch_product<F>(acc[r][t], xh[t], xl[t], wb[r], sb[r]);
+					__builtin_amdgcn_sched_barrier(0);
+					if constexpr ((j + 1) % PB == 0)
+					{
+#pragma unroll
+						for (int r = 0; r < RT; ++r)
+							rows.load(s_w + (q * RT + r) * 1024, scale[q][r], r, (b_lo + i0 + j + 1 - PB + WB) / PB, p_hi);
+					}
+					__builtin_amdgcn_sched_barrier(0);
+				};
+				block(std::integral_constant<int, 0>{});
+				block(std::integral_constant<int, 1>{});
+				if constexpr (U >= 4)
+				{
+					block(std::integral_constant<int, 2>{});
+					block(std::integral_constant<int, 3>{});
+				}
+				if constexpr (U == 8)
+				{
+					block(std::integral_constant<int, 4>{});
+					block(std::integral_constant<int, 5>{});
+					block(std::integral_constant<int, 6>{});
+					block(std::integral_constant<int, 7>{});
+				}
+			}
+			if constexpr (F == kGemvQ4S)
+			{
+				for (int st = kg; st < (nb + 31) / 32; st += 2)
+#pragma unroll
+					for (int r = 0; r < RT; ++r)
+					{
+						const bf16x8 b = bias_operand(rows.bi[r], 32 * st + 8 * grp, nb);
+#pragma unroll
+						for (int t = 0; t < TT; ++t)
+						{
+							const u32x4* xs = reinterpret_cast<const u32x4*>(
+								                  x_sums(p, st, min(tt * TT + t, p.x_tiles - 1))) + lane;
+#pragma unroll
+							for (int i = 2; i >= 0; --i) acc[r][t] = mfma16x16x32(as_bf16x8(xs[64 * i]), b, acc[r][t]);
+						}
+					}
+			}
+
+			// (the blocks after the last are in flight, as zeros, into LDS)
+			wait_loads<0>();
+			__syncthreads();
+			f32x4* s_sum = reinterpret_cast<f32x4*>(s_raw) + wr * RT * TT * 64 + lane;
+			if (kg == 1)
+			{
+#pragma unroll
+				for (int r = 0; r < RT; ++r)
+#pragma unroll
+					for (int t = 0; t < TT; ++t) s_sum[(r * TT + t) * 64] = acc[r][t];
+			}
+			__syncthreads();
+			if (kg == 0)
+			{
+#pragma unroll
+				for (int r = 0; r < RT; ++r)
+				{
+					const int row = row0 + 16 * r + col;
+					if (row >= p.rows) continue;
+					const mat_row mr = locate(p, row);
+#pragma unroll
+					for (int t = 0; t < TT; ++t)
+					{
+						const f32x4 v = acc[r][t] + s_sum[(r * TT + t) * 64];
+#pragma unroll
+						for (int i = 0; i < 4; ++i)
+						{
+							const int tok = (tt * TT + t) * 16 + 4 * grp + i;
+							if (tok < p.n_batch) mr.m.y[tok * mr.m.y_stride + mr.r] = v[i];
+						}
+					}
 				}
 			}
 		}
@@ -726,6 +1396,61 @@ namespace nnchip
 				mr.m.y[t * mr.m.y_stride + mr.r] = s;
 			}
 		}
+
+		template <int F, int RT, int TT>
+		void launch_batch(const gemv_params& p, hipStream_t stream)
+		{
+			const size_t lds = static_cast<size_t>(kBatchWaves) * RT * std::max(TT, kBatchDepth<F, RT, TT>) * 1024;
+			gemv_batch_kernel<F, RT, TT><<<(p.rows + 16 * RT - 1) / (16 * RT), 64 * kBatchWaves, lds, stream>>>(p);
+		}
+
+		template <int F, int RT, int TT, int WR, int SLOTS, int NPW>
+		void launch_tile(const gemv_params& p, hipStream_t stream)
+		{
+			using S = tile_shape<F, RT, TT, WR, SLOTS, NPW>;
+			const int n_tt = (p.x_tiles + TT - 1) / TT, n_rt = (p.rows + 16 * RT * WR - 1) / (16 * RT * WR);
+			gemv_tile_kernel<F, RT, TT, WR, SLOTS, NPW><<<(n_rt + 7) / 8 * 8 * n_tt, 128 * WR, S::kLds, stream>>>(p);
+		}
+
+		// 17 vectors and more. A row's sums do not depend on the choices by
+		// `rows` below, only on the columns and the number of vectors, so the
+		// matrices of a group get the bits of their own calls.
+		template <int F>
+		void launch_wide(const gemv_params& p, hipStream_t stream)
+		{
+			const int nb = p.cols / 32, items = (F == kGemvQ4S ? (nb + 31) & ~31 : nb) * p.x_tiles;
+			gemv_stage_x_kernel<F><<<(items + 3) / 4, 256, 0, stream>>>(p);
+			if (p.n_batch <= 64)
+			{
+				// Two 16-row tiles per work-group halve the reads of X; one
+				// fills more CUs (from 160 work-groups on, two).
+				const bool two = p.rows >= 32 * 160;
+				if (p.n_batch <= 32)
+					two ? launch_batch<F, 2, 2>(p, stream) : launch_batch<F, 1, 2>(p, stream);
+				else
+					two ? launch_batch<F, 2, 4>(p, stream) : launch_batch<F, 1, 4>(p, stream);
+				return;
+			}
+			// rows x vectors per work-group, by what fills the 256 CUs (us, BF16 /
+			// Q8_0): 128 x 128 moves the fewest bytes per product but takes one
+			// CU each (6144 x 2560, 512 vectors, 192 of them: 48.1 / 61.3 against
+			// 54.5 / 63.8 in 128 x 64; 19456 x 2560, 608 of them: 133 / 161
+			// against 131 / 154); 64 x 64 for few (6144 x 2560, 128 vectors, 96
+			// work-groups of 128 x 64: 31.0 / 34.0 against 34.8 / 40.7); and for
+			// BF16 the deeper rings, one work-group per CU, where there is no
+			// second one to cover the waits (2560 x 4096, 512 vectors: 45.4
+			// against 49.5; with 384 work-groups 62.0 against 54.5).
+			const long long w128 = 1LL * ((p.rows + 127) / 128) * ((p.x_tiles + 7) / 8);
+			const long long w64 = 1LL * ((p.rows + 127) / 128) * ((p.x_tiles + 3) / 4);
+			if (w128 >= 128 && w128 <= 256)
+				launch_tile<F, 2, 8, 4, 2, 2>(p, stream);
+			else if (w64 <= 128)
+				launch_tile<F, 2, 4, 2, 2, 2>(p, stream);
+			else if (F == kGemvBf16 && w64 <= 256)
+				launch_tile<kGemvBf16, 2, 4, 4, 4, 4>(p, stream);
+			else
+				launch_tile<F, 2, 4, 4, 2, 2>(p, stream);
+		}
 	}
 
 	void gemv_plan(int rows, int cols, int n_batch, int format, int& n_split, int& split_blocks)
@@ -740,6 +1465,12 @@ namespace nnchip
 			++max_blocks;
 		n_split = (nb + max_blocks - 1) / max_blocks;
 		split_blocks = (nb + n_split - 1) / n_split;
+	}
+
+	size_t gemv_staged_bytes(int cols, int n_batch, int format)
+	{
+		const size_t nb = cols / 32, tiles = (n_batch + 15) / 16;
+		return tiles * (nb * 2048 + (format == kGemvQ4S ? (nb + 31) / 32 * 3072 : 0));
 	}
 
 	int gemv_vec_groups(int rows)
@@ -774,6 +1505,16 @@ namespace nnchip
 			case kGemvBf16: gemv_vec_kernel<kGemvBf16><<<grid, 256, lds, stream>>>(p); return true;
 			case kGemvQ8_0: gemv_vec_kernel<kGemvQ8_0><<<grid, 256, lds, stream>>>(p); return true;
 			case kGemvQ4S: gemv_vec_kernel<kGemvQ4S><<<grid, 256, lds, stream>>>(p); return true;
+			default: return false;
+			}
+		}
+		if (p.xs)
+		{
+			switch (p.format)
+			{
+			case kGemvBf16: launch_wide<kGemvBf16>(p, stream); return true;
+			case kGemvQ8_0: launch_wide<kGemvQ8_0>(p, stream); return true;
+			case kGemvQ4S: launch_wide<kGemvQ4S>(p, stream); return true;
 			default: return false;
 			}
 		}

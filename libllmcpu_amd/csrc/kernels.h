@@ -176,9 +176,13 @@ namespace nnchip
 	bool launch_fill_normal(void* dst, uint64_t n, uint64_t seed, int norm_dim, bool bf16, hipStream_t stream);
 
 	// The weight gemvs (reference nn_ops.h:95-180): Y[t] = W . X[t] for
-	// t < n_batch <= 16, W in one of nnc's three weight layouts.
+	// t < n_batch, W in one of nnc's three weight layouts.
 	constexpr int kGemvBf16 = 0, kGemvQ8_0 = 1, kGemvQ4S = 2;
-	constexpr int kGemvMaxBatch = 16;
+	constexpr int kGemvMaxBatch = 16; // vectors of one gemv_kernel launch
+	// Vectors of one launch with staged X (gemv_params::xs), and the bytes its
+	// staging may take (32-bit offsets).
+	constexpr int kGemvWideBatch = 1024;
+	constexpr size_t kGemvStagedMax = size_t{1} << 30;
 	constexpr size_t kGemvLdsBudget = 64 << 10; // dynamic LDS per one-vector gemv work-group
 	// The batch kernel: weight rows per work-group (16 per wavefront) and its
 	// dynamic LDS budget per weight layout (at most two work-groups per CU),
@@ -224,6 +228,11 @@ namespace nnchip
 		int mrow[kGemvMaxMats + 1];
 		const float* x; // [n_batch] vectors of cols floats, x_stride apart
 		const float* xsum; // Q4_S: [n_batch] runs of cols / 32 block sums, xsum_stride apart; or null
+		// X as matrix operands (gemv_staged_bytes; written by the launch's first
+		// kernel), which more than kGemvMaxBatch vectors need; null: the other
+		// kernels, which read x itself.
+		void* xs;
+		int x_tiles; // tiles of 16 vectors
 		float* part; // [n_split][n_batch][rows] partial sums when n_split > 1 (stacked rows)
 		size_t x_stride, xsum_stride;
 		int rows, cols, n_batch; // rows: all matrices' rows
@@ -237,6 +246,9 @@ namespace nnchip
 
 	// K splits for a (rows, cols) gemv of n_batch vectors.
 	void gemv_plan(int rows, int cols, int n_batch, int format, int& n_split, int& split_blocks);
+
+	// Bytes of a call's staged X.
+	size_t gemv_staged_bytes(int cols, int n_batch, int format);
 
 	bool launch_gemv(const gemv_params& p, hipStream_t stream);
 

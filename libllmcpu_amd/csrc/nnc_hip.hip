@@ -185,7 +185,7 @@ struct nnc_hip_kv
 	dev_scratch part; // decode partials
 	dev_scratch q; // device copies of host q / gate and append rows
 	dev_scratch gate;
-	dev_scratch gemv_part; // weight gemv partial sums over K splits
+	dev_scratch gemv_part; // weight gemvs: partial sums over K splits, or X staged as operands
 	int* n_bad = nullptr; // per buffer: elements of V's fp16 copy now marked kF16Bad (device)
 	unsigned* counts = nullptr; // kFuseCounts arrival counts of the fused decode merge (device, zero between calls)
 	dev_scratch rows_k;
@@ -1079,10 +1079,26 @@ namespace
 		p.rows = acc;
 	}
 
+	// Whether a gemv of n_batch vectors runs with staged X: more than
+	// kGemvMaxBatch of them, and the scratch holds the staging or may grow (not
+	// while the stream is captured into a graph, where nothing can be
+	// allocated: then kGemvMaxBatch vectors at a time, as without it).
+	static bool gemv_wide(nnc_hip_kv* kv, uint32_t cols, uint32_t n_batch, int format)
+	{
+		if (n_batch <= nnchip::kGemvMaxBatch) return false;
+		const size_t bytes = nnchip::gemv_staged_bytes(
+			static_cast<int>(cols), static_cast<int>(std::min<uint32_t>(n_batch, nnchip::kGemvWideBatch)), format);
+		if (bytes > nnchip::kGemvStagedMax) return false;
+		if (bytes <= kv->gemv_part.bytes) return true;
+		hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+		return hipStreamIsCapturing(kv->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+	}
+
 	// Weight gemvs over the same X on the context's stream: one launch per
-	// chunk of at most kGemvMaxBatch vectors for all the matrices together
-	// (stacked along the rows), or one per matrix when a matrix other than
-	// the last has a row count that is not a multiple of 16.
+	// chunk of at most kGemvWideBatch vectors (kGemvMaxBatch without staged X)
+	// for all the matrices together (stacked along the rows), or one per
+	// matrix when a matrix other than the last has a row count that is not a
+	// multiple of 16.
 	static nnc_status gemv_impl(nnc_hip_kv* kv, int format, int n_mat, const nnc_hip_gemv_mat* mats, const float* X,
 	                     size_t x_stride, const float* XSUM, size_t xsum_stride, uint32_t cols, uint32_t n_batch)
 	{
@@ -1125,14 +1141,25 @@ namespace
 		}
 		uint32_t rows[nnchip::kGemvMaxMats];
 		for (int m = 0; m < n_mat; ++m) rows[m] = mats[m].rows;
-		for (uint32_t t0 = 0; t0 < n_batch; t0 += nnchip::kGemvMaxBatch)
+		const bool wide = gemv_wide(kv, cols, n_batch, format);
+		const uint32_t chunk = wide ? nnchip::kGemvWideBatch : nnchip::kGemvMaxBatch;
+		for (uint32_t t0 = 0; t0 < n_batch; t0 += chunk)
 		{
-			const int nb = static_cast<int>(std::min<uint32_t>(n_batch - t0, nnchip::kGemvMaxBatch));
+			const int nb = static_cast<int>(std::min<uint32_t>(n_batch - t0, chunk));
 			nnchip::gemv_params p{};
 			p.format = format;
 			stack_rows(p, rows, n_mat);
 			int n_split = 1, split_blocks = 1;
-			nnchip::gemv_plan(p.rows, static_cast<int>(cols), nb, format, n_split, split_blocks);
+			if (wide && nb > nnchip::kGemvMaxBatch)
+			{
+				if (nnc_status s = reserve(kv, kv->gemv_part,
+				                           nnchip::gemv_staged_bytes(static_cast<int>(cols), nb, format), "gemv scratch"))
+					return s;
+				p.xs = kv->gemv_part.ptr;
+				p.x_tiles = (nb + 15) / 16;
+			}
+			else
+				nnchip::gemv_plan(p.rows, static_cast<int>(cols), nb, format, n_split, split_blocks);
 			if (n_split > 1)
 				if (nnc_status s = reserve(kv, kv->gemv_part,
 				                           static_cast<size_t>(n_split) * nb * static_cast<size_t>(p.rows) * sizeof(float),

@@ -509,3 +509,102 @@ def test_hip_gemv_argmax_row0_nan(orc, rows):
         print(f"case argmax {rows} x 256, row 0 NaN", flush=True)
         got, want = kv.gemv_argmax(w, x), orc.gemv_bf16_argmax(w, x)
         assert got == want if rows % 4 != 0 else argmax_ok(w, x, got, want)
+
+
+# More than 16 vectors run with X staged as matrix operands: 17-64 (one and
+# two 16-row tiles per work-group) and more (the four tile shapes, chosen by
+# the number of work-groups), and past 1024 in chunks. Odd rows, an odd number
+# of 32-column blocks, fewer blocks than a loop pass, a last chunk of 1 and of 6.
+WIDE_SHAPES = [
+    (33, 32, 17), (1000, 96, 32), (5136, 160, 33), (5136, 416, 64), (72, 2560, 20),
+    (40, 64, 65), (129, 1056, 70), (4112, 672, 100), (9000, 352, 129), (16400, 96, 200), (2000, 224, 1030), (16, 32, 1025),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,n", WIDE_SHAPES, ids=[f"{r}x{c}x{n}" for r, c, n in WIDE_SHAPES])
+def test_hip_gemv_many_vectors(orc, rows, cols, n):
+    """Each layout against its weights in float64, to the 1e-5 * sum |w x| bound
+    of the smaller batches (X as bf16 hi + lo is off by at most 2^-17 of it);
+    Q4_S with the caller's block sums gives the same bits; a group the bits of
+    its matrices' own calls."""
+    import libllmcpu_amd as nh
+    from libllmcpu_amd import hip_rt
+
+    rng = np.random.default_rng(rows * 7 + cols + n)
+    wf = (rng.standard_normal((rows, cols)) * 0.05).astype(np.float32)
+    x = (rng.standard_normal((n, cols)) * 2).astype(np.float32)
+    with nh.KVCache([16], [64]) as kv:
+        for fmt, wl in layouts(orc, wf).items():
+            print(f"case gemv {fmt} {rows} x {cols}, {n} vectors", flush=True)
+            got = kv.gemv(fmt, wl, x, rows=rows, cols=cols)
+            pick = np.unique(np.r_[0, 15, 16, n // 2, n - 1])
+            want = oracle_gemv(orc, fmt, wl, np.ascontiguousarray(x[pick]))
+            err = np.abs(got[pick].astype(np.float64) - want)
+            b = bound(fmt, wl, x[pick])
+            print(f"  max |err| / bound {float((err / b).max()):.3f}", flush=True)
+            assert np.all(err <= b), fmt
+            # every vector: the same vectors in another order, row by row the same bits
+            order = rng.permutation(n)
+            again = kv.gemv(fmt, wl, np.ascontiguousarray(x[order]), rows=rows, cols=cols)
+            if n <= 1024:  # (one launch: a vector's bits do not depend on its place)
+                assert np.array_equal(again.view(np.uint32), got[order].view(np.uint32)), fmt
+            if fmt == "q4_s":
+                got2 = kv.gemv(fmt, wl, x, rows=rows, cols=cols, xsum=orc.block_sums(x))
+                assert np.array_equal(got2, got)
+            if rows % 16 == 0:  # the matrix twice in one group
+                dev = [hip_rt.malloc(a.nbytes) for a in (*wl, x)] + [hip_rt.malloc(2 * n * rows * 4)]
+                try:
+                    for d, a in zip(dev, (*wl, x)):
+                        hip_rt.to_device(d, a)
+                    w, y = tuple(dev[:len(wl)]), dev[-1]
+                    kv.gemv_group_device(fmt, [(w, y, rows), (w, y + 4 * n * rows, rows)], dev[len(wl)], cols=cols, n_batch=n)
+                    kv.sync()
+                    both = hip_rt.to_host(np.empty((2, n, rows), np.float32), y)
+                    assert np.array_equal(both[0].view(np.uint32), got.view(np.uint32)), fmt
+                    assert np.array_equal(both[1].view(np.uint32), got.view(np.uint32)), fmt
+                finally:
+                    for d in dev:
+                        hip_rt.free(d)
+
+
+@pytest.mark.gpu
+def test_hip_gemv_many_vectors_in_a_graph(orc):
+    """Captured by a cache whose scratch has not grown (nothing can be
+    allocated then), a long batch runs 16 vectors at a time; replays of the
+    graph give each time what the same launches give eagerly, and within the
+    bound what the staged path gives."""
+    import libllmcpu_amd as nh
+    from libllmcpu_amd import hip_rt
+
+    rows, cols, n = 96, 512, 40  # (one K split: 16 vectors need no scratch)
+    rng = np.random.default_rng(3)
+    wl = layouts(orc, (rng.standard_normal((rows, cols)) * 0.05).astype(np.float32))["bf16"]
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    dev = [hip_rt.malloc(a.nbytes) for a in (*wl, x)] + [hip_rt.malloc(n * rows * 4)]
+    try:
+        for d, a in zip(dev, (*wl, x)):
+            hip_rt.to_device(d, a)
+        with nh.KVCache([16], [64]) as kv:
+            print("case gemv of 40 vectors under capture", flush=True)
+            call = lambda: kv.gemv_device("bf16", (dev[0],), dev[1], dev[2], rows=rows, cols=cols, n_batch=n)  # noqa: E731
+            g = hip_rt.Graph(kv.stream, call)
+            first = None
+            for _ in range(3):
+                hip_rt.to_device(dev[2], np.zeros((n, rows), np.float32))
+                g.launch(kv.stream)
+                kv.sync()
+                got = hip_rt.to_host(np.empty((n, rows), np.float32), dev[2])
+                first = got if first is None else first
+                assert np.array_equal(got, first)
+            g.close()
+            for t in range(0, n, 16):
+                m = min(16, n - t)
+                assert np.array_equal(kv.gemv("bf16", wl, x[t:t + m], rows=rows, cols=cols), first[t:t + m])
+            call()
+            kv.sync()
+            wide = hip_rt.to_host(np.empty((n, rows), np.float32), dev[2])
+            assert np.all(np.abs(wide.astype(np.float64) - first) <= 2 * bound("bf16", wl, x))
+    finally:
+        for d in dev:
+            hip_rt.free(d)
