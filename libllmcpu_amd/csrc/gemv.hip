@@ -43,6 +43,9 @@ namespace nnchip
 		// Qwen3-4B layer 86.9 -> 77.8 us; the quantised layouts, whose loads are
 		// 8 and 4 bytes, ran 8 % slower that way: 92.1 and 94.5 us).
 		constexpr int kGemvBf16Blocks = 16;
+		// The quantised layouts' blocks per K split, what gemv_batch_lds holds
+		// of 16 vectors.
+		constexpr int kGemvQuantBlocks = 18;
 		// 16-byte loads in flight per lane of the one-vector kernel, per layout
 		// (a one-vector Qwen3-4B layer, us, at 8 / 6 / 4: BF16 55.7 / 56.1 /
 		// 59.2, Q8_0 48.7 / 48.9 / 48.4, Q4_S 51.5 / 50.9 / 48.4; 16 slower).
@@ -319,14 +322,15 @@ namespace nnchip
 			}
 		}
 
-		// ---- 17 vectors and more: gemv_batch_kernel and gemv_tile_kernel ----
+		// ---- gemv_batch_kernel and gemv_tile_kernel ----
 		//
 		// X is split into bf16 hi + lo once per call (gemv_stage_x_kernel) and
 		// the products go the other way round: A = X (16 vectors x 32 columns),
 		// B = the rows' weights, so D holds vectors 4 (l / 16) + i of row
 		// l % 16: a row's scale is one value per lane and Y's rows are
-		// consecutive lanes. Batches of 512 vectors ran 16 at a time through
-		// gemv_kernel before, the weights read 32 times over.
+		// consecutive lanes. (512 vectors ran 16 at a time through gemv_kernel
+		// before, the weights read 32 times over: 6144 x 2560 BF16 448 us, now
+		// 47.)
 
 		// 64 bytes of each of 16 weight rows per wavefront load (a "piece", 16
 		// bytes per lane: row l % 16, bytes 16 (l / 16) ..): this many 32-column
@@ -610,11 +614,6 @@ namespace nnchip
 		}
 
 		constexpr int kBatchWaves = 8;
-		// Pieces in flight per wavefront (their X with them: loads complete in
-		// order, so X fetched any later would wait for every W load before it).
-		template <int F, int RT, int TT>
-		constexpr int kBatchDepth = F == kGemvBf16 ? (TT == 2 ? 4 : 2) : F == kGemvQ8_0 ? (TT == 2 ? 2 : 1) : 1;
-
 		// Y[t][r] for 16 RT rows per work-group and up to 16 TT vectors, W
 		// streamed once. The wavefronts split the columns (contiguous runs of
 		// whole pieces, the same whatever RT and the number of rows, so a row
@@ -624,13 +623,16 @@ namespace nnchip
 		// vectors x 32 columns, bf16 hi + lo), B = the rows' weights, so D holds
 		// vectors 4 (l / 16) + i of row l % 16: a row's scale is one value per
 		// lane, and Y's rows are consecutive lanes. X comes as operands
-		// (gemv_stage_x_kernel).
+		// (gemv_stage_x_kernel). Bound by latency at small sizes and by the
+		// wavefronts' short lives at large ones, so one piece at a time and many
+		// wavefronts: rings of 2, 4 and 6 pieces ran 16 vectors of 6144 x 2560
+		// (BF16 / Q8_0 / Q4_S) in 14.2 / 13.2 / 14.3, 14.7 / 16.0 / 23.1 and 15.0 /
+		// 15.0 / - us against 13.0 / 12.4 / 13.2, and 16 wavefronts in 14.8 / 13.2 /
+		// 13.5.
 		template <int F, int RT, int TT>
 		__global__ __launch_bounds__(64 * kBatchWaves) void gemv_batch_kernel(const gemv_params p)
 		{
-			constexpr int PB = kPieceBlocks<F>, D = kBatchDepth<F, RT, TT>;
-			// Loads of one piece: X's, the weights' and their scales'.
-			constexpr int NL = 2 * PB * TT + RT * (F == kGemvBf16 ? 1 : 2);
+			constexpr int PB = kPieceBlocks<F>;
 			extern __shared__ __attribute__((aligned(16))) unsigned char s_raw[];
 			const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 			const int grp = lane >> 4;
@@ -638,17 +640,14 @@ namespace nnchip
 			const int i_lo = wave * np / kBatchWaves, i_hi = (wave + 1) * np / kBatchWaves;
 			const int row0 = blockIdx.x * 16 * RT;
 			const batch_rows<F, RT> rows(p, row0);
-			unsigned char* const s_w = s_raw + wave * D * RT * 1024; // [D][RT] pieces of this wavefront
+			unsigned char* const s_w = s_raw + wave * RT * 1024; // [RT] pieces of this wavefront
 
-			struct piece_t
-			{
-				u32x4 xh[PB][TT], xl[PB][TT];
-				uint32_t scale[RT];
-			} ring[D];
+			u32x4 xh[PB][TT], xl[PB][TT];
+			uint32_t scale[RT];
 			const uint32_t xs_block = static_cast<uint32_t>(p.x_tiles) * 2048u;
 			const __amdgpu_buffer_rsrc_t rx =
 				__builtin_amdgcn_make_buffer_rsrc(x_staged(p, min(i_lo * PB, nb - 1), 0), 0, 0x7fffffff, 0x00020000);
-			auto load = [&](piece_t& k, int d, int i) __attribute__((always_inline))
+			auto load = [&](int i) __attribute__((always_inline))
 			{
 #pragma unroll
 				for (int j = 0; j < PB; ++j)
@@ -659,12 +658,12 @@ namespace nnchip
 #pragma unroll
 					for (int t = 0; t < TT; ++t)
 					{
-						k.xh[j][t] = __builtin_amdgcn_raw_buffer_load_b128(rx, o, 2048 * t, 0);
-						k.xl[j][t] = __builtin_amdgcn_raw_buffer_load_b128(rx, o, 2048 * t + 1024, 0);
+						xh[j][t] = __builtin_amdgcn_raw_buffer_load_b128(rx, o, 2048 * t, 0);
+						xl[j][t] = __builtin_amdgcn_raw_buffer_load_b128(rx, o, 2048 * t + 1024, 0);
 					}
 				}
 #pragma unroll
-				for (int r = 0; r < RT; ++r) rows.load(s_w + (d * RT + r) * 1024, k.scale[r], r, i, i_hi);
+				for (int r = 0; r < RT; ++r) rows.load(s_w + r * 1024, scale[r], r, i, i_hi);
 			};
 
 			f32x4 acc[RT][TT];
@@ -673,41 +672,29 @@ namespace nnchip
 #pragma unroll
 				for (int t = 0; t < TT; ++t) acc[r][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-#pragma unroll
-			for (int d = 0; d < D; ++d)
+			load(i_lo);
+			for (int i = i_lo; i < i_hi; ++i)
 			{
-				load(ring[d], d, i_lo + d);
-				__builtin_amdgcn_sched_barrier(0);
-			}
-			for (int i0 = i_lo; i0 < i_hi; i0 += D)
-			{
+				wait_loads<0>();
+				bf16x8 wb[RT][PB];
+				float sc[RT][4];
 #pragma unroll
-				for (int d = 0; d < D; ++d)
+				for (int r = 0; r < RT; ++r)
 				{
-					piece_t& k = ring[d];
-					wait_loads<(D - 1) * NL>(); // this piece's have landed
-					bf16x8 wb[RT][PB];
-					float sc[RT][4];
-#pragma unroll
-					for (int r = 0; r < RT; ++r)
-					{
-						batch_operands<F>(rows.read(s_w + (d * RT + r) * 1024), wb[r]);
-						batch_scales<F>(k.scale[r], sc[r]);
-					}
-#pragma unroll
-					for (int j = 0; j < PB; ++j)
-#pragma unroll
-						for (int t = 0; t < TT; ++t)
-#pragma unroll
-							for (int r = 0; r < RT; ++r)
-								batch_product<F>(acc[r][t], as_bf16x8(k.xh[j][t]), as_bf16x8(k.xl[j][t]), wb[r][j], sc[r][j]);
-					// (kept in this order, or the scheduler gathers the loads at
-					// the loop's end and the next piece waits for all of them;
-					// the piece's LDS reads have returned: the products took them)
-					__builtin_amdgcn_sched_barrier(0);
-					load(k, d, i0 + d + D);
-					__builtin_amdgcn_sched_barrier(0);
+					batch_operands<F>(rows.read(s_w + r * 1024), wb[r]);
+					batch_scales<F>(scale[r], sc[r]);
 				}
+#pragma unroll
+				for (int j = 0; j < PB; ++j)
+#pragma unroll
+					for (int t = 0; t < TT; ++t)
+#pragma unroll
+						for (int r = 0; r < RT; ++r)
+							batch_product<F>(acc[r][t], as_bf16x8(xh[j][t]), as_bf16x8(xl[j][t]), wb[r][j], sc[r][j]);
+				// (the piece's LDS reads have returned: the products took them)
+				__builtin_amdgcn_sched_barrier(0);
+				load(i + 1);
+				__builtin_amdgcn_sched_barrier(0);
 			}
 			wait_loads<0>(); // (zeros on their way to LDS)
 			__syncthreads(); // the sums take the pieces' place
@@ -1400,8 +1387,8 @@ namespace nnchip
 		template <int F, int RT, int TT>
 		void launch_batch(const gemv_params& p, hipStream_t stream)
 		{
-			const size_t lds = static_cast<size_t>(kBatchWaves) * RT * std::max(TT, kBatchDepth<F, RT, TT>) * 1024;
-			gemv_batch_kernel<F, RT, TT><<<(p.rows + 16 * RT - 1) / (16 * RT), 64 * kBatchWaves, lds, stream>>>(p);
+			gemv_batch_kernel<F, RT, TT><<<(p.rows + 16 * RT - 1) / (16 * RT), 64 * kBatchWaves,
+			                               kBatchWaves * RT * TT * 1024, stream>>>(p);
 		}
 
 		template <int F, int RT, int TT, int WR, int SLOTS, int NPW>
@@ -1412,7 +1399,7 @@ namespace nnchip
 			gemv_tile_kernel<F, RT, TT, WR, SLOTS, NPW><<<(n_rt + 7) / 8 * 8 * n_tt, 128 * WR, S::kLds, stream>>>(p);
 		}
 
-		// 17 vectors and more. A row's sums do not depend on the choices by
+		// The calls with staged X. A row's sums do not depend on the choices by
 		// `rows` below, only on the columns and the number of vectors, so the
 		// matrices of a group get the bits of their own calls.
 		template <int F>
@@ -1425,7 +1412,9 @@ namespace nnchip
 				// Two 16-row tiles per work-group halve the reads of X; one
 				// fills more CUs (from 160 work-groups on, two).
 				const bool two = p.rows >= 32 * 160;
-				if (p.n_batch <= 32)
+				if (p.n_batch <= 16)
+					two ? launch_batch<F, 2, 1>(p, stream) : launch_batch<F, 1, 1>(p, stream);
+				else if (p.n_batch <= 32)
 					two ? launch_batch<F, 2, 2>(p, stream) : launch_batch<F, 1, 2>(p, stream);
 				else
 					two ? launch_batch<F, 2, 4>(p, stream) : launch_batch<F, 1, 4>(p, stream);
@@ -1453,18 +1442,34 @@ namespace nnchip
 		}
 	}
 
-	void gemv_plan(int rows, int cols, int n_batch, int format, int& n_split, int& split_blocks)
+	void gemv_plan(int cols, int n_batch, int format, int& n_split, int& split_blocks)
 	{
-		(void)rows;
 		const int nb = cols / 32;
-		// As few K splits as the LDS copy of X^T allows (one for a single
-		// vector at every nnc shape), the splits equal in size.
+		// As few K splits as the LDS copy of X^T of 16 vectors allows, the
+		// splits equal in size (fewer vectors leave room for longer splits,
+		// whose few work-groups ran 2 vectors of 2560 x 9728 in 38 us where 16
+		// took 23).
 		int max_blocks = 1;
-		const int cap = format == kGemvBf16 ? kGemvBf16Blocks : nb;
+		const int cap = format == kGemvBf16 ? kGemvBf16Blocks : kGemvQuantBlocks;
 		while (max_blocks < std::min(nb, cap) && gemv_lds_bytes(max_blocks + 1, n_batch) <= gemv_batch_lds(format))
 			++max_blocks;
 		n_split = (nb + max_blocks - 1) / max_blocks;
 		split_blocks = (nb + n_split - 1) / n_split;
+	}
+
+	// Up to 16 vectors run either kernel. One stream / three at once, 16 vectors,
+	// us, gemv_kernel against gemv_batch_kernel (with its staging): Q8_0 6144 x
+	// 2560 16.4 / 10.1 against 12.6 / 9.1, 2560 x 4096 15.8 / 8.8, 11.7 / 8.6,
+	// 19456 x 2560 29.6 / 22.5, 27.8 / 19.0, 3072 x 2048 15.4 / 8.6, 8.4 / 7.4,
+	// but 2560 x 9728 23.3 / 13.2, 23.5 / 18.6 (X is read once per 16 rows
+	// there, four times the weights' bytes); BF16 3072 x 2048 12.7 / 8.4, 9.5 /
+	// 7.3, but 19456 x 2560 29.4 / 23.3, 33 / -. The lines are at numbers of
+	// columns, not of rows, so that a matrix gets the same bits alone and in a
+	// group.
+	bool gemv_stages_x(int cols, int n_batch, int format)
+	{
+		if (gemv_vec_fits(cols, n_batch, format)) return false;
+		return n_batch > kGemvMaxBatch || cols <= (format == kGemvBf16 ? 2048 : 6144);
 	}
 
 	size_t gemv_staged_bytes(int cols, int n_batch, int format)

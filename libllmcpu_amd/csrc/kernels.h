@@ -229,8 +229,8 @@ namespace nnchip
 		const float* x; // [n_batch] vectors of cols floats, x_stride apart
 		const float* xsum; // Q4_S: [n_batch] runs of cols / 32 block sums, xsum_stride apart; or null
 		// X as matrix operands (gemv_staged_bytes; written by the launch's first
-		// kernel), which more than kGemvMaxBatch vectors need; null: the other
-		// kernels, which read x itself.
+		// kernel) where gemv_stages_x; null: the other kernels, which read x
+		// itself.
 		void* xs;
 		int x_tiles; // tiles of 16 vectors
 		float* part; // [n_split][n_batch][rows] partial sums when n_split > 1 (stacked rows)
@@ -244,10 +244,12 @@ namespace nnchip
 		int first_sticks; // 1: the result is 0 when y[0] is NaN (the reference's linear scan from y[0])
 	};
 
-	// K splits for a (rows, cols) gemv of n_batch vectors.
-	void gemv_plan(int rows, int cols, int n_batch, int format, int& n_split, int& split_blocks);
+	// K splits of gemv_kernel.
+	void gemv_plan(int cols, int n_batch, int format, int& n_split, int& split_blocks);
 
-	// Bytes of a call's staged X.
+	// Whether a call runs with its X staged (gemv_params::xs), and the bytes that
+	// takes.
+	bool gemv_stages_x(int cols, int n_batch, int format);
 	size_t gemv_staged_bytes(int cols, int n_batch, int format);
 
 	bool launch_gemv(const gemv_params& p, hipStream_t stream);

@@ -1079,26 +1079,37 @@ namespace
 		p.rows = acc;
 	}
 
-	// Whether a gemv of n_batch vectors runs with staged X: more than
-	// kGemvMaxBatch of them, and the scratch holds the staging or may grow (not
-	// while the stream is captured into a graph, where nothing can be
-	// allocated: then kGemvMaxBatch vectors at a time, as without it).
-	static bool gemv_wide(nnc_hip_kv* kv, uint32_t cols, uint32_t n_batch, int format)
+	// Scratch of one launch of nb vectors: X staged as matrix operands, or the
+	// K splits' partial sums.
+	static size_t gemv_scratch_bytes(int rows, int cols, int nb, int format)
 	{
-		if (n_batch <= nnchip::kGemvMaxBatch) return false;
-		const size_t bytes = nnchip::gemv_staged_bytes(
-			static_cast<int>(cols), static_cast<int>(std::min<uint32_t>(n_batch, nnchip::kGemvWideBatch)), format);
-		if (bytes > nnchip::kGemvStagedMax) return false;
-		if (bytes <= kv->gemv_part.bytes) return true;
-		hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-		return hipStreamIsCapturing(kv->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+		if (nnchip::gemv_vec_fits(cols, nb, format)) return 0;
+		if (nnchip::gemv_stages_x(cols, nb, format)) return nnchip::gemv_staged_bytes(cols, nb, format);
+		int n_split, split_blocks;
+		nnchip::gemv_plan(cols, nb, format, n_split, split_blocks);
+		return n_split > 1 ? static_cast<size_t>(n_split) * nb * static_cast<size_t>(rows) * sizeof(float) : 0;
+	}
+
+	// Vectors per launch of a gemv of n_batch: all of them up to kGemvWideBatch;
+	// while the stream is captured into a graph and the scratch would have to
+	// grow (nothing can be allocated then), one, on the one-vector kernel.
+	static uint32_t gemv_chunk(const nnc_hip_kv* kv, int rows, int cols, uint32_t n_batch, int format)
+	{
+		if (n_batch == 1) return 1;
+		const int nb = static_cast<int>(std::min<uint32_t>(n_batch, nnchip::kGemvWideBatch));
+		if (nnchip::gemv_staged_bytes(cols, nb, format) > nnchip::kGemvStagedMax) return nnchip::kGemvMaxBatch;
+		if (gemv_scratch_bytes(rows, cols, nb, format) > kv->gemv_part.bytes && nnchip::gemv_vec_fits(cols, 1, format))
+		{
+			hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+			if (hipStreamIsCapturing(kv->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone) return 1;
+		}
+		return nnchip::kGemvWideBatch;
 	}
 
 	// Weight gemvs over the same X on the context's stream: one launch per
-	// chunk of at most kGemvWideBatch vectors (kGemvMaxBatch without staged X)
-	// for all the matrices together (stacked along the rows), or one per
-	// matrix when a matrix other than the last has a row count that is not a
-	// multiple of 16.
+	// chunk of gemv_chunk vectors for all the matrices together (stacked along
+	// the rows), or one per matrix when a matrix other than the last has a row
+	// count that is not a multiple of 16.
 	static nnc_status gemv_impl(nnc_hip_kv* kv, int format, int n_mat, const nnc_hip_gemv_mat* mats, const float* X,
 	                     size_t x_stride, const float* XSUM, size_t xsum_stride, uint32_t cols, uint32_t n_batch)
 	{
@@ -1141,30 +1152,24 @@ namespace
 		}
 		uint32_t rows[nnchip::kGemvMaxMats];
 		for (int m = 0; m < n_mat; ++m) rows[m] = mats[m].rows;
-		const bool wide = gemv_wide(kv, cols, n_batch, format);
-		const uint32_t chunk = wide ? nnchip::kGemvWideBatch : nnchip::kGemvMaxBatch;
+		const uint32_t chunk = gemv_chunk(kv, static_cast<int>(total), static_cast<int>(cols), n_batch, format);
 		for (uint32_t t0 = 0; t0 < n_batch; t0 += chunk)
 		{
 			const int nb = static_cast<int>(std::min<uint32_t>(n_batch - t0, chunk));
 			nnchip::gemv_params p{};
 			p.format = format;
 			stack_rows(p, rows, n_mat);
-			int n_split = 1, split_blocks = 1;
-			if (wide && nb > nnchip::kGemvMaxBatch)
+			p.n_split = 1;
+			p.split_blocks = static_cast<int>(cols / 32);
+			if (const size_t bytes = gemv_scratch_bytes(p.rows, static_cast<int>(cols), nb, format))
+				if (nnc_status s = reserve(kv, kv->gemv_part, bytes, "gemv scratch")) return s;
+			if (nnchip::gemv_stages_x(static_cast<int>(cols), nb, format))
 			{
-				if (nnc_status s = reserve(kv, kv->gemv_part,
-				                           nnchip::gemv_staged_bytes(static_cast<int>(cols), nb, format), "gemv scratch"))
-					return s;
 				p.xs = kv->gemv_part.ptr;
 				p.x_tiles = (nb + 15) / 16;
 			}
-			else
-				nnchip::gemv_plan(p.rows, static_cast<int>(cols), nb, format, n_split, split_blocks);
-			if (n_split > 1)
-				if (nnc_status s = reserve(kv, kv->gemv_part,
-				                           static_cast<size_t>(n_split) * nb * static_cast<size_t>(p.rows) * sizeof(float),
-				                           "gemv scratch"))
-					return s;
+			else if (!nnchip::gemv_vec_fits(static_cast<int>(cols), nb, format))
+				nnchip::gemv_plan(static_cast<int>(cols), nb, format, p.n_split, p.split_blocks);
 			for (int m = 0; m < n_mat; ++m)
 			{
 				const nnc_hip_gemv_mat& M = mats[m];
@@ -1177,8 +1182,6 @@ namespace
 			p.xsum_stride = xsum_stride;
 			p.cols = static_cast<int>(cols);
 			p.n_batch = nb;
-			p.n_split = n_split;
-			p.split_blocks = split_blocks;
 			if (!nnchip::launch_gemv(p, kv->stream)) return fail(NNC_ERR_UNSUPPORTED_MODEL, "gemv format %d", format);
 			NNC_HIP_TRY(hipGetLastError(), "gemv launch");
 		}
