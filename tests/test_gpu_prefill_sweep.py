@@ -52,3 +52,27 @@ def test_prefill_sweep(orc, case):
     ea, er = errors(got, want)
     say(f"  max-abs {ea:.3e} max-rel {er:.3e}")
     assert ea <= 5e-3
+
+
+@pytest.mark.parametrize("n_tok,group,n_kv", ((256, 4, 8), (257, 4, 8), (320, 4, 8), (600, 1, 16), (130, 8, 8)))
+def test_prefill_hd64_both_register_budgets(orc, n_tok, group, n_kv):
+    """head_dim 64 runs four wavefronts per SIMD in launches of more than 128
+    work-groups of 64 rows (256 tokens of group 4 over 8 KV heads are 128), two in smaller
+    ones: both sides of the line, with V's copy and (a value beyond its limit) without it."""
+    cfg = synth.AttnConfig(60, "hd64", group * n_kv, n_kv, 64, 1)
+    n_seq = n_tok + 77
+    K, V = synth.cache_buffer(cfg, 0, n_seq, n_seq)
+    q = synth.qk_rows(cfg, 0, 0, np.arange(77, n_seq), cfg.n_head)
+    kw = dict(n_head=cfg.n_head, n_kv=n_kv, head_dim=64, scale=cfg.attn_scale)
+    for big in (False, True):
+        if big:
+            V = V.copy()
+            V[3, 5] = nh.bf16_round(np.array([10.0], np.float32))[0]
+        say(f"case hd64 {n_tok} tokens, group {group}, n_kv {n_kv}, V beyond its copy's limit: {big}")
+        with nh.KVCache([n_seq], [cfg.kv_dim]) as kv:
+            kv.append(0, 0, K, V)
+            got = kv.attend(0, q, pos0=77, n_seq=n_seq, **kw)
+        want = orc.attend_layer(q, K, V, kv_bf16=True, rows=n_seq, pos0=77, n_seq=n_seq, **kw)
+        ea, er = errors(got, want)
+        say(f"  max-abs {ea:.3e} max-rel {er:.3e}")
+        assert ea <= 5e-3
