@@ -77,17 +77,20 @@ namespace nnchip
 				return *reinterpret_cast<const float4*>(static_cast<const float*>(base) + elem);
 		}
 
-		// The keys of row block `blk` (its 64 rows' spans together: both ends
-		// of a span move forward with the position) and its splits: split z
-		// covers keys b_lo + z * split_keys .. + split_keys - 1, relative to
-		// the block's first key, so a block has (b_hi - b_lo) / split_keys + 1
-		// of them and the grid's z extent is the largest such count.
+		// The keys of row block `blk` of BLOCK rows (its rows' spans together:
+		// both ends of a span move forward with the position; the first key
+		// rounded down to a multiple of ALIGN) and its splits: split z covers
+		// keys b_lo + z * split_keys .. + split_keys - 1, relative to the block's
+		// first key, so a block has (b_hi - b_lo) / split_keys + 1 of them and
+		// the grid's z extent is the largest such count.
+		template <int BLOCK = kTileBlock, int ALIGN = 1>
 		__device__ __forceinline__ void tiled_block_keys(const decode_params& p, int G, int blk, int& b_lo, int& b_hi)
 		{
-			const int n_rows = p.n_tok * G, r0 = blk * kTileBlock, r1 = min(r0 + kTileBlock, n_rows) - 1;
+			const int n_rows = p.n_tok * G, r0 = blk * BLOCK, r1 = min(r0 + BLOCK, n_rows) - 1;
 			int unused;
 			attn_span(p.causal, p.window, p.pos0 + r0 / G, p.n_seq, b_lo, unused);
 			attn_span(p.causal, p.window, p.pos0 + r1 / G, p.n_seq, unused, b_hi);
+			b_lo = b_lo / ALIGN * ALIGN;
 		}
 
 		__device__ __forceinline__ int tiled_block_splits(int b_lo, int b_hi, int split_keys)
@@ -308,13 +311,14 @@ namespace nnchip
 		// 2^(m_z - M), l likewise; out = o * (1 / l), 0 when l == 0. Four rows
 		// per work-group, 64 threads per row, four elements per thread and
 		// pass.
+		template <int BLOCK, int ALIGN>
 		__global__ __launch_bounds__(256) void tiled_merge_kernel(const decode_params p, int hd, int G)
 		{
 			const int n_rows = p.n_tok * G, r = blockIdx.x * 4 + (threadIdx.x >> 6), kvh = blockIdx.y;
 			if (r >= n_rows) return;
 			const int lane = threadIdx.x & 63, t = r / G, h = r % G;
 			int b_lo, b_hi, first, last;
-			tiled_block_keys(p, G, r / kTileBlock, b_lo, b_hi);
+			tiled_block_keys<BLOCK, ALIGN>(p, G, r / BLOCK, b_lo, b_hi);
 			attn_span(p.causal, p.window, p.pos0 + t, p.n_seq, first, last);
 			const int z0 = first <= last ? (first - b_lo) / p.split_keys : 0;
 			const int z1 = first <= last ? (last - b_lo) / p.split_keys : -1;
@@ -348,6 +352,355 @@ namespace nnchip
 			}
 		}
 
+		// ---- F32 caches at head_dim 64, 128 and 256, long batches: tiled3_kernel ----
+		//
+		// fp32 products as sums of bf16 ones: x = x1 + x2 + x3, three bf16 that
+		// hold fp32's 24 bits, and x . y = x1y1 + (x1y2 + x2y1) + (x1y3 + x2y2 +
+		// x3y1); the three products left out are below 2^-25 of x . y, half of
+		// one fp32 rounding. Six bf16 MFMAs of 32 deep take 96 clocks where the
+		// fp32 ones take 256 (v_mfma_f32_16x16x4_f32: 157 TFLOP/s on this part,
+		// and the kernel above is bound by them). Sums stay fp32, and a 32-deep
+		// MFMA rounds its sum less often than eight 4-deep ones: against 64 bits
+		// (relative, 2-norm) a 2048-token embedding call is off by 4.6e-7 (fp32
+		// MFMAs: 5.7e-7), 1000 causal tokens of 4 x 256 by 4.7e-7 (5.8e-7), 300
+		// over 1500 keys of 16 x 128 by 4.4e-7 (4.6e-7).
+		//
+		// tiled3_split_kernel first writes the span's K and V as operands (kept
+		// for the call; every row block reads them): per 32-key group and KV head
+		// 1 KB fragments in lane order, K [16-key tile][32 elements][part], V
+		// [16 elements][part] with the keys in the score registers' order. A
+		// work-group takes 128 rows; Q (three parts) and O stay in registers. A
+		// group's K and V have one LDS buffer each: the next K loads (LDS-DMA)
+		// during this group's P . V, the next V during the next scores. us, one
+		// stream / three at once, tiled_kernel -> this: six layers of a 2048-token
+		// embedding call (five windowed) 408 / 318 -> 340 / 220, four of 1000
+		// causal tokens of 4 x 256 244 / 171 -> 197 / 123, two of 300 tokens over
+		// 1500 keys of 16 x 128 133 / 90 -> 119 / 63. Bound by the matrix cores,
+		// and in a windowed layer (four groups per work-group) by Q's staging,
+		// the operands' kernel and the merge around them.
+		constexpr int kT3Block = kTiled3Block, kT3Keys = kTiled3Keys;
+
+		__device__ __forceinline__ void split3(const float (&x)[8], u32x4 (&out)[3])
+		{
+#pragma unroll
+			for (int j = 0; j < 4; ++j)
+			{
+				const float a = x[2 * j], b = x[2 * j + 1];
+				const uint32_t h = cvt_pk_bf16(a, b);
+				const float a1 = a - bf16_lo(h), b1 = b - bf16_hi(h);
+				const uint32_t m = cvt_pk_bf16(a1, b1);
+				out[0][j] = h;
+				out[1][j] = m;
+				out[2][j] = cvt_pk_bf16(a1 - bf16_lo(m), b1 - bf16_hi(m));
+			}
+		}
+
+		// Bytes of a group's K (or V) of one head.
+		template <int HD>
+		constexpr uint32_t kT3Bytes = HD * kT3Keys * 6;
+
+		// Group g0 + blockIdx.x of head blockIdx.y; keys outside k_lo .. k_hi as
+		// zeros.
+		template <int HD>
+		__global__ __launch_bounds__(256) void tiled3_split_kernel(const decode_params p, char* split, int k_lo, int k_hi, int g0)
+		{
+			const int kvh = blockIdx.y, key0 = (g0 + static_cast<int>(blockIdx.x)) * kT3Keys;
+			char* dst = split + (static_cast<size_t>(kvh) * gridDim.x + blockIdx.x) * 2 * kT3Bytes<HD>;
+			const size_t head_off = static_cast<size_t>(kvh) * HD;
+			auto row = [&](int k) { return static_cast<size_t>(k % p.rows) * p.kv_dim + head_off; };
+			const float* K = static_cast<const float*>(p.K);
+			const float* V = static_cast<const float*>(p.V);
+			for (int i = threadIdx.x; i < HD * 4; i += 256) // (8 elements each)
+			{
+				const int lane = i & 63, f = i >> 6, r = lane & 15, g = lane >> 4;
+				float x[8];
+				u32x4 o[3];
+				{
+					const int t = f / (HD / 32), kk = f % (HD / 32), k = key0 + 16 * t + r;
+					float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
+					if (k >= k_lo && k <= k_hi)
+					{
+						const float* s = K + row(k) + 32 * kk + 8 * g;
+						a = *reinterpret_cast<const float4*>(s);
+						b = *reinterpret_cast<const float4*>(s + 4);
+					}
+					x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
+					x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
+					split3(x, o);
+#pragma unroll
+					for (int c = 0; c < 3; ++c) *reinterpret_cast<u32x4*>(dst + (f * 3 + c) * 1024 + 16 * lane) = o[c];
+				}
+				{
+#pragma unroll
+					for (int j = 0; j < 8; ++j)
+					{
+						const int k = key0 + 16 * (j >> 2) + 4 * g + (j & 3);
+						x[j] = k >= k_lo && k <= k_hi ? V[row(k) + 16 * f + r] : 0.0f;
+					}
+					split3(x, o);
+#pragma unroll
+					for (int c = 0; c < 3; ++c)
+						*reinterpret_cast<u32x4*>(dst + kT3Bytes<HD> + (f * 3 + c) * 1024 + 16 * lane) = o[c];
+				}
+			}
+		}
+
+		__device__ __forceinline__ void t3_dma(__amdgpu_buffer_rsrc_t r, unsigned char* dst, uint32_t off, uint32_t s_off)
+		{
+			typedef __attribute__((address_space(3))) void* lds_ptr;
+			__builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)dst, 16, off, s_off, 0, 0);
+		}
+
+		// At most N of this wavefront's loads in flight (s_waitcnt vmcnt(N), the
+		// other counters not waited on), then everyone's.
+		template <int N>
+		__device__ __forceinline__ void t3_wait_barrier()
+		{
+			static_assert(N < 16, "vmcnt");
+			__builtin_amdgcn_sched_barrier(0);
+			__builtin_amdgcn_s_waitcnt(0x0F70 | N);
+			__builtin_amdgcn_s_barrier();
+			__builtin_amdgcn_sched_barrier(0);
+		}
+
+		// This wavefront's LDS reads have returned (lgkmcnt(0)), then everyone's.
+		__device__ __forceinline__ void t3_read_barrier()
+		{
+			__builtin_amdgcn_sched_barrier(0);
+			__builtin_amdgcn_s_waitcnt(0xC07F);
+			__builtin_amdgcn_s_barrier();
+			__builtin_amdgcn_sched_barrier(0);
+		}
+
+		// c[y][x] += a[x] . b[y] of three-part operands, the smallest products
+		// first, the sums in turn (a sum's next product waits for its last).
+		template <int NA>
+		__device__ __forceinline__ void mfma3(const u32x4 (&a)[2][3], const u32x4 (&b)[NA][3], f32x4 (&c)[NA][2])
+		{
+			constexpr int A[6] = {2, 0, 1, 1, 0, 0}, B[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+			for (int u = 0; u < 6; ++u)
+#pragma unroll
+				for (int x = 0; x < 2; ++x)
+#pragma unroll
+					for (int y = 0; y < NA; ++y) c[y][x] = mfma16x16x32(as_bf16x8(a[x][A[u]]), as_bf16x8(b[y][B[u]]), c[y][x]);
+		}
+
+		// Row tiles per wavefront: two at head_dim 64 and 128 (a fragment read
+		// from LDS serves two products; four wavefronts, two work-groups per
+		// CU), one at 256, where two tiles' Q and O left one wavefront per SIMD and
+		// spilled (417 / 278 us for the embedding call above; eight wavefronts,
+		// two per SIMD, 340 / 220).
+		template <int HD>
+		constexpr int kT3Tiles = HD == 256 ? 1 : 2;
+
+		template <int HD>
+		__global__ __launch_bounds__(512 / kT3Tiles<HD>) __attribute__((amdgpu_waves_per_eu(2, 2))) void tiled3_kernel(
+			const decode_params p, const char* split, int G, int g0, int n_g)
+		{
+			constexpr int NA = kT3Tiles<HD>, NWV = 8 / NA;
+			constexpr int KK = HD / 32, DT = HD / 16, ND = kT3Bytes<HD> / 1024 / NWV; // DMAs per wavefront per K (or V)
+			__shared__ __attribute__((aligned(16))) unsigned char s_k[kT3Bytes<HD>];
+			__shared__ __attribute__((aligned(16))) unsigned char s_v[kT3Bytes<HD>];
+			const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+			const int c = lane >> 4, r16 = lane & 15;
+			const int kvh = blockIdx.y, z = blockIdx.z, n_rows = p.n_tok * G;
+
+			int b_lo, b_hi;
+			tiled_block_keys<kT3Block, kT3Keys>(p, G, blockIdx.x, b_lo, b_hi);
+			if (z >= tiled_block_splits(b_lo, b_hi, p.split_keys)) return; // the whole work-group: no split here
+			const int w_lo = b_lo + z * p.split_keys, w_hi = min(b_hi, w_lo + p.split_keys - 1);
+			const int n_steps = (w_hi - w_lo) / kT3Keys + 1;
+
+			const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+				const_cast<char*>(split) + static_cast<size_t>(kvh) * n_g * 2 * kT3Bytes<HD>, 0,
+				static_cast<int>(static_cast<uint32_t>(n_g) * 2 * kT3Bytes<HD>), 0x00020000);
+			// K (v = 0) or V (1) of step st; a step past the last loads nothing
+			// (zeros), so that the counts of loads in flight stay the same.
+			auto load = [&](int st, int v, unsigned char* dst) __attribute__((always_inline))
+			{
+				const uint32_t o = st < n_steps ? (static_cast<uint32_t>(w_lo / kT3Keys - g0 + st) * 2 + v) * kT3Bytes<HD> : 0u;
+				const uint32_t lo = st < n_steps ? 16u * lane + 1024u * wave : 0x80000000u;
+#pragma unroll
+				for (int u = 0; u < ND; ++u) t3_dma(rs, dst + 1024 * (NWV * u + wave), lo, o + 1024 * NWV * u);
+			};
+			load(0, 0, s_k);
+			load(0, 1, s_v);
+
+			// This lane's row of each of the wavefront's tiles.
+			int r_lo[NA], r_hi[NA];
+			size_t qo[NA];
+			u32x4 q[KK][NA][3];
+#pragma unroll
+			for (int a = 0; a < NA; ++a)
+			{
+				const int row = blockIdx.x * kT3Block + 16 * (NA * wave + a) + r16;
+				const bool ok = row < n_rows;
+				const int t = ok ? row / G : 0, h = ok ? row % G : 0;
+				int first, last;
+				attn_span(p.causal, p.window, p.pos0 + t, p.n_seq, first, last);
+				r_lo[a] = ok ? max(first, w_lo) : 1;
+				r_hi[a] = ok ? min(last, w_hi) : 0;
+				qo[a] = (static_cast<size_t>(t) * p.n_head + static_cast<size_t>(kvh) * G + h) * HD;
+#pragma unroll
+				for (int kk = 0; kk < KK; ++kk)
+				{
+					const float4 u = *reinterpret_cast<const float4*>(p.q + qo[a] + 32 * kk + 8 * c);
+					const float4 v = *reinterpret_cast<const float4*>(p.q + qo[a] + 32 * kk + 8 * c + 4);
+					const float x[8] = {u.x * p.qscale, u.y * p.qscale, u.z * p.qscale, u.w * p.qscale,
+					                    v.x * p.qscale, v.y * p.qscale, v.z * p.qscale, v.w * p.qscale};
+					split3(x, q[kk][a]);
+				}
+			}
+
+			f32x4 acc[DT / 2][NA][2]; // elements 32 d + 16 x + 4 c + i
+			float m_run[NA], l_run[NA];
+#pragma unroll
+			for (int a = 0; a < NA; ++a)
+			{
+				m_run[a] = -INFINITY;
+				l_run[a] = 0.0f;
+#pragma unroll
+				for (int d = 0; d < DT / 2; ++d) acc[d][a][0] = acc[d][a][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+			}
+			// (Q's loads came after the first DMAs: none of this is counted on)
+			__builtin_amdgcn_sched_barrier(0);
+			__builtin_amdgcn_s_waitcnt(0x0F70);
+
+			for (int st = 0; st < n_steps; ++st)
+			{
+				const int k0 = w_lo + st * kT3Keys;
+				t3_wait_barrier<ND>(); // K has landed; V may be in flight
+				// S^T: tile t's keys k0 + 16 t + 4 c + i of row r16.
+				f32x4 sc[NA][2];
+#pragma unroll
+				for (int a = 0; a < NA; ++a) sc[a][0] = sc[a][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+				// (the next fragments are read before the current ones' products)
+				u32x4 f[2][2][3];
+				auto read_k = [&](int kk, u32x4 (&o)[2][3]) __attribute__((always_inline))
+				{
+#pragma unroll
+					for (int t = 0; t < 2; ++t)
+#pragma unroll
+						for (int u = 0; u < 3; ++u)
+							o[t][u] = *reinterpret_cast<const u32x4*>(s_k + ((t * KK + kk) * 3 + u) * 1024 + 16 * lane);
+				};
+				read_k(0, f[0]);
+#pragma unroll
+				for (int kk = 0; kk < KK; ++kk)
+				{
+					if (kk + 1 < KK) read_k(kk + 1, f[(kk + 1) & 1]);
+					__builtin_amdgcn_sched_barrier(0);
+					mfma3<NA>(f[kk & 1], q[kk], sc);
+					__builtin_amdgcn_sched_barrier(0);
+				}
+				t3_read_barrier(); // everyone is done with K
+				load(st + 1, 0, s_k);
+
+				// Online softmax of each row (offset, weights and their sum as in
+				// tiled_kernel); P as the B operand: k-slot 4 t + i.
+				u32x4 pw[NA][3];
+#pragma unroll
+				for (int a = 0; a < NA; ++a)
+				{
+					float cmax = -INFINITY;
+#pragma unroll
+					for (int t = 0; t < 2; ++t)
+#pragma unroll
+						for (int i = 0; i < 4; ++i)
+						{
+							const int k = k0 + 16 * t + 4 * c + i;
+							sc[a][t][i] = (k >= r_lo[a] && k <= r_hi[a]) ? sc[a][t][i] : -INFINITY;
+							cmax = fmaxf(cmax, sc[a][t][i]);
+						}
+					cmax = row4_max(cmax);
+					const bool raise = cmax > m_run[a] + kTileLazy;
+					if (__builtin_amdgcn_ballot_w64(raise))
+					{
+						const float alpha = raise && m_run[a] != -INFINITY ? fast_exp2(m_run[a] - cmax) : 1.0f;
+						m_run[a] = raise ? cmax : m_run[a];
+						l_run[a] *= alpha;
+#pragma unroll
+						for (int d = 0; d < DT / 2; ++d)
+						{
+							acc[d][a][0] *= alpha;
+							acc[d][a][1] *= alpha;
+						}
+					}
+					const float m_use = m_run[a] == -INFINITY ? 0.0f : m_run[a];
+					float w[8], ls = 0.0f;
+#pragma unroll
+					for (int j = 0; j < 8; ++j)
+					{
+						w[j] = fast_exp2(sc[a][j >> 2][j & 3] - m_use);
+						ls += w[j];
+					}
+					l_run[a] += row4_sum(ls);
+					split3(w, pw[a]);
+				}
+
+				t3_wait_barrier<ND>(); // V has landed; the next K may be in flight
+				auto read_v = [&](int d, u32x4 (&o)[2][3]) __attribute__((always_inline))
+				{
+#pragma unroll
+					for (int t = 0; t < 2; ++t)
+#pragma unroll
+						for (int u = 0; u < 3; ++u)
+							o[t][u] = *reinterpret_cast<const u32x4*>(s_v + ((d + t) * 3 + u) * 1024 + 16 * lane);
+				};
+				read_v(0, f[0]);
+#pragma unroll
+				for (int d = 0; d < DT; d += 2)
+				{
+					if (d + 2 < DT) read_v(d + 2, f[(d / 2 + 1) & 1]);
+					__builtin_amdgcn_sched_barrier(0);
+					mfma3<NA>(f[(d / 2) & 1], pw, acc[d / 2]);
+					__builtin_amdgcn_sched_barrier(0);
+				}
+				t3_read_barrier(); // everyone is done with V
+				load(st + 1, 1, s_v);
+			}
+			__builtin_amdgcn_sched_barrier(0);
+			__builtin_amdgcn_s_waitcnt(0x0F70); // (zeros on their way to LDS)
+
+#pragma unroll
+			for (int a = 0; a < NA; ++a)
+			{
+				const int row = blockIdx.x * kT3Block + 16 * (NA * wave + a) + r16;
+				if (row >= n_rows) continue;
+				if (p.n_split > 1)
+				{
+					float* gp = tiled_partial(p, G, HD, row / G, kvh, z, row % G);
+#pragma unroll
+					for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4*>(gp + 16 * d + 4 * c) = acc[d / 2][a][d & 1];
+					if (c == 0) *reinterpret_cast<float2*>(gp + HD) = make_float2(m_run[a], l_run[a]);
+				}
+				else
+				{
+					const float inv = l_run[a] > 0.0f ? 1.0f / l_run[a] : 0.0f;
+#pragma unroll
+					for (int d = 0; d < DT; ++d)
+					{
+						const size_t oi = qo[a] + 16 * d + 4 * c;
+						float4 o;
+						o.x = gated(acc[d / 2][a][d & 1][0] * inv, p.gate, oi);
+						o.y = gated(acc[d / 2][a][d & 1][1] * inv, p.gate, oi + 1);
+						o.z = gated(acc[d / 2][a][d & 1][2] * inv, p.gate, oi + 2);
+						o.w = gated(acc[d / 2][a][d & 1][3] * inv, p.gate, oi + 3);
+						*reinterpret_cast<float4*>(p.out + oi) = o;
+					}
+				}
+			}
+		}
+
+		template <int HD>
+		void launch_t3(const decode_params& p, int G, void* split, int k_lo, int k_hi, int g0, dim3 sgrid, dim3 grid,
+		               hipStream_t stream)
+		{
+			tiled3_split_kernel<HD><<<sgrid, 256, 0, stream>>>(p, static_cast<char*>(split), k_lo, k_hi, g0);
+			tiled3_kernel<HD><<<grid, 512 / kT3Tiles<HD>, 0, stream>>>(p, static_cast<const char*>(split), G, g0, sgrid.x);
+		}
+
 		template <int HD, int HDMAX>
 		void launch_hd(const decode_params& p, int n_tok, int head_dim, int group, bool bf16, hipStream_t stream)
 		{
@@ -379,7 +732,24 @@ namespace nnchip
 				launch_hd<0, 512>(p, n_tok, head_dim, group, bf16, stream);
 		}
 		if (p.n_split > 1)
-			tiled_merge_kernel<<<dim3((n_tok * group + 3) / 4, p.n_kv), 256, 0, stream>>>(p, head_dim, group);
+			tiled_merge_kernel<kTileBlock, 1><<<dim3((n_tok * group + 3) / 4, p.n_kv), 256, 0, stream>>>(p, head_dim, group);
+		return true;
+	}
+
+	bool launch_tiled3(const decode_params& p, int n_tok, int head_dim, int group, void* split, int k_lo, int k_hi,
+	                   hipStream_t stream)
+	{
+		const int g0 = k_lo / kT3Keys, n_g = k_hi / kT3Keys - g0 + 1;
+		const dim3 sgrid(n_g, p.n_kv), grid((n_tok * group + kT3Block - 1) / kT3Block, p.n_kv, p.n_split);
+		switch (head_dim)
+		{
+		case 64: launch_t3<64>(p, group, split, k_lo, k_hi, g0, sgrid, grid, stream); break;
+		case 128: launch_t3<128>(p, group, split, k_lo, k_hi, g0, sgrid, grid, stream); break;
+		case 256: launch_t3<256>(p, group, split, k_lo, k_hi, g0, sgrid, grid, stream); break;
+		default: return false;
+		}
+		if (p.n_split > 1)
+			tiled_merge_kernel<kT3Block, kT3Keys><<<dim3((n_tok * group + 3) / 4, p.n_kv), 256, 0, stream>>>(p, head_dim, group);
 		return true;
 	}
 }

@@ -107,6 +107,23 @@ namespace nnchip
 	}
 	bool launch_tiled(const decode_params& p, int n_tok, int head_dim, int group, bool bf16, hipStream_t stream);
 
+	// The same batches of F32 caches at head_dim 64, 128 and 256 with the
+	// products as sums of six bf16 ones (24 bits): the span's K and V (keys
+	// k_lo .. k_hi) are first written to `split` as matrix operands,
+	// tiled3_bytes of them. Row blocks of 128, splits of a multiple of 32 keys
+	// relative to the block's first key rounded down to 32.
+	constexpr int kTiled3Block = 128, kTiled3Keys = 32;
+	__host__ __device__ inline bool tiled3_shape(int head_dim)
+	{
+		return head_dim == 64 || head_dim == 128 || head_dim == 256;
+	}
+	inline size_t tiled3_bytes(int k_lo, int k_hi, int n_kv, int head_dim)
+	{
+		return static_cast<size_t>(k_hi / kTiled3Keys - k_lo / kTiled3Keys + 1) * n_kv * head_dim * kTiled3Keys * 12;
+	}
+	bool launch_tiled3(const decode_params& p, int n_tok, int head_dim, int group, void* split, int k_lo, int k_hi,
+	                   hipStream_t stream);
+
 	// Tiled MFMA attention for a batch of query tokens.
 	struct prefill_params
 	{

@@ -402,6 +402,8 @@ namespace
 		int sk;
 		bool tiled = false; // the tiled fp32-MFMA kernel instead of the per-token split-K kernels
 		int nz = 0; // tiled: splits of the row block with the most keys (sk keys each, from the block's first key)
+		size_t split_bytes = 0; // tiled, not 0: tiled3_kernel, K and V of keys k_lo .. k_hi as operands in so much scratch
+		int k_lo = 0, k_hi = 0;
 	};
 
 	// Bytes of the tiled kernel's partials for a plan entry (none for one split).
@@ -441,17 +443,20 @@ namespace
 	// src (already checked to hold them) or to the cache's scratch.
 	// One launch of the tiled kernel (plan entry d: its tokens, split size
 	// and split count), partials in src or the cache's scratch.
+	// (Scratch: the operands of tiled3_kernel, then the partials.)
 	nnc_status tiled_launch(nnc_hip_kv* kv, const kv_buffer& b, const float* q, float* out, const float* gate,
 	                        const decode_plan& d, int32_t pos0, int32_t n_seq, int32_t window, bool causal, int32_t n_head,
 	                        int32_t n_kv, int32_t head_dim, float scale, const part_source& src)
 	{
-		const size_t bytes = tiled_part_bytes(d, n_head, n_kv, head_dim);
+		const size_t bytes = d.split_bytes + tiled_part_bytes(d, n_head, n_kv, head_dim);
 		float* part = src.ptr;
 		if (!part && bytes)
 		{
 			if (nnc_status s = reserve(kv, kv->part, bytes, "tiled scratch")) return s;
 			part = static_cast<float*>(kv->part.ptr);
 		}
+		void* split = part;
+		if (part) part += d.split_bytes / sizeof(float);
 		nnchip::decode_params p{};
 		p.q = q;
 		p.out = out;
@@ -471,7 +476,8 @@ namespace
 		p.split_keys = d.sk;
 		p.n_split = d.nz;
 		p.qscale = scale * 1.4426950408889634f;
-		if (!nnchip::launch_tiled(p, d.n, head_dim, n_head / n_kv, kv->bf16, kv->stream))
+		if (d.split_bytes ? !nnchip::launch_tiled3(p, d.n, head_dim, n_head / n_kv, split, d.k_lo, d.k_hi, kv->stream)
+		                  : !nnchip::launch_tiled(p, d.n, head_dim, n_head / n_kv, kv->bf16, kv->stream))
 			return fail(NNC_ERR_UNSUPPORTED_MODEL, "no tiled kernel for head_dim %d, group %d", head_dim, n_head / n_kv);
 		NNC_HIP_TRY(hipGetLastError(), "tiled launch");
 		return NNC_OK;
@@ -580,39 +586,88 @@ namespace
 		}
 	}
 
-	// The tiled kernel's launches: chunks of at most kTiledChunk tokens. Each
-	// row block of 64 (token, head) rows splits its keys (the union of its
+	// Most scratch of one tiled3_kernel launch, operands and partials: what the
+	// no-alloc entry point's array holds, so that it runs the same launches.
+	constexpr size_t kTiled3Scratch = NNC_HIP_NOALLOC_SCRATCH_BYTES;
+
+	// The tiled kernels' launches: chunks of at most kTiledChunk tokens. Each
+	// row block of (token, head) rows splits its keys (the union of its
 	// rows' spans) into splits of sk keys from its first key; sk is chosen so
 	// that the work-groups of the launch about fill the part once (the
-	// kernel's resident work-groups per CU: 4 up to head_dim 128, 2 up to
-	// 256, else 1), at least 64 keys per split.
+	// kernel's resident work-groups per CU: tiled_kernel 4 up to head_dim 128,
+	// 2 up to 256, else 1; tiled3_kernel 1 at head_dim 256, else 2), at least
+	// 64 keys per split.
+	// tiled3_kernel takes the F32 chunks of its head shapes from 512 rows per
+	// KV head on, since writing the operands costs a pass over the keys whatever
+	// the rows, and 4000 rows in all, since under that its three launches and
+	// 128-row blocks leave the chip idle (four layers of 3 x 256, three of them
+	// windowed, us, one stream / three, tiled_kernel -> it: 300 tokens, 900 rows,
+	// 98 / 50 -> 123 / 55; 700 132 / 71 -> 149 / 70; 1024 162 / 85 -> 157 / 98;
+	// 1344, 4032 rows, 183 / 107 -> 169 / 91; 1700 196 / 125 -> 186 / 104; causal
+	// layers of 1000 tokens of 4 x 256, 4000 rows, 244 / 171 -> 197 / 123), as far
+	// as its scratch goes: kTiled3Scratch, and while the stream is captured
+	// (nothing can be allocated) what is there.
 	void plan_tiled(const nnc_hip_kv* kv, int32_t n_tok, int32_t pos0, int32_t n_seq, int32_t window, bool causal,
-	                int32_t n_kv, int32_t head_dim, int group, std::vector<decode_plan>& plan)
+	                int32_t n_kv, int32_t head_dim, int group, const part_source& src, std::vector<decode_plan>& plan)
 	{
-		const int per_cu = head_dim <= 128 ? 4 : head_dim <= 256 ? 2 : 1;
 		for (int32_t t0 = 0; t0 < n_tok; t0 += kTiledChunk)
 		{
 			const int32_t nt = std::min(kTiledChunk, n_tok - t0);
-			const long long n_rows = static_cast<long long>(nt) * group, n_blk = (n_rows + 63) / 64;
-			std::vector<int> spans(static_cast<size_t>(n_blk));
-			int max_span = 1;
-			for (long long blk = 0; blk < n_blk; ++blk)
+			const long long n_rows = static_cast<long long>(nt) * group;
+			auto make = [&](int block, int align, int per_cu, long long max_splits)
 			{
-				const long long r0 = 64 * blk, r1 = std::min(r0 + 64, n_rows) - 1;
-				int lo, hi, unused;
-				nnchip::attn_span(causal ? 1 : 0, window, pos0 + t0 + static_cast<int32_t>(r0 / group), n_seq, lo, unused);
-				nnchip::attn_span(causal ? 1 : 0, window, pos0 + t0 + static_cast<int32_t>(r1 / group), n_seq, unused, hi);
-				spans[static_cast<size_t>(blk)] = std::max(0, hi - lo + 1);
-				max_span = std::max(max_span, hi - lo + 1);
+				const long long n_blk = (n_rows + block - 1) / block;
+				std::vector<int> spans(static_cast<size_t>(n_blk));
+				int max_span = 1;
+				for (long long blk = 0; blk < n_blk; ++blk)
+				{
+					const long long r0 = block * blk, r1 = std::min(r0 + block, n_rows) - 1;
+					int lo, hi, unused;
+					nnchip::attn_span(causal ? 1 : 0, window, pos0 + t0 + static_cast<int32_t>(r0 / group), n_seq, lo, unused);
+					nnchip::attn_span(causal ? 1 : 0, window, pos0 + t0 + static_cast<int32_t>(r1 / group), n_seq, unused, hi);
+					lo = lo / align * align;
+					spans[static_cast<size_t>(blk)] = std::max(0, hi - lo + 1);
+					max_span = std::max(max_span, hi - lo + 1);
+				}
+				const long long want =
+					std::min(max_splits, std::max<long long>(1, 1LL * kv->n_cu * per_cu / (n_blk * n_kv)));
+				const int step = std::max(align, 16);
+				long long sk = (max_span + want - 1) / want;
+				sk = std::max<long long>(64, (sk + step - 1) / step * step);
+				int nz = 1;
+				for (int sp : spans)
+					if (sp > 0) nz = std::max(nz, static_cast<int>((sp - 1) / sk + 1));
+				return decode_plan{t0, nt, static_cast<int>(sk), true, nz};
+			};
+			if (!kv->bf16 && nnchip::tiled3_shape(head_dim) && n_rows >= 512 && n_rows * n_kv >= 4000)
+			{
+				int k_lo, k_hi, unused;
+				nnchip::attn_span(causal ? 1 : 0, window, pos0 + t0, n_seq, k_lo, unused);
+				nnchip::attn_span(causal ? 1 : 0, window, pos0 + t0 + nt - 1, n_seq, unused, k_hi);
+				const size_t split = k_hi >= k_lo ? nnchip::tiled3_bytes(k_lo, k_hi, n_kv, head_dim) : kTiled3Scratch + 1;
+				if (split <= kTiled3Scratch)
+				{
+					const size_t row_bytes = static_cast<size_t>(n_rows) * n_kv * (head_dim + 4) * sizeof(float); // per split
+					const long long room = static_cast<long long>((kTiled3Scratch - split) / row_bytes);
+					decode_plan d = make(nnchip::kTiled3Block, nnchip::kTiled3Keys, head_dim == 256 ? 1 : 2,
+					                     std::max<long long>(room, 1));
+					d.split_bytes = split;
+					d.k_lo = k_lo;
+					d.k_hi = k_hi;
+					const size_t need = split + tiled_part_bytes(d, group * n_kv, n_kv, head_dim);
+					hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+					const bool there = src.ptr ? need <= src.bytes
+					                           : need <= kv->part.bytes ||
+					                                 (hipStreamIsCapturing(kv->stream, &st) == hipSuccess &&
+					                                  st == hipStreamCaptureStatusNone);
+					if (need <= kTiled3Scratch && there)
+					{
+						plan.push_back(d);
+						continue;
+					}
+				}
 			}
-			const long long want = std::max<long long>(1, 1LL * kv->n_cu * per_cu / (n_blk * n_kv));
-			long long sk = (max_span + want - 1) / want;
-			sk = std::max<long long>(64, (sk + 15) / 16 * 16);
-			int nz = 1;
-			for (int sp : spans)
-				if (sp > 0) nz = std::max(nz, static_cast<int>((sp - 1) / sk + 1));
-			decode_plan d{t0, nt, static_cast<int>(sk), true, nz};
-			plan.push_back(d);
+			plan.push_back(make(64, 1, head_dim <= 128 ? 4 : head_dim <= 256 ? 2 : 1, LLONG_MAX));
 		}
 	}
 
@@ -670,7 +725,7 @@ namespace
 			return NNC_OK;
 		}
 		else if (tiled)
-			plan_tiled(kv, n_tok, pos0, n_seq, window, causal, n_kv, head_dim, group, plan);
+			plan_tiled(kv, n_tok, pos0, n_seq, window, causal, n_kv, head_dim, group, src, plan);
 		else
 			plan_f32_chunks(kv, n_tok, pos0, n_seq, window, causal, n_kv, head_dim, group, plan);
 
@@ -680,7 +735,7 @@ namespace
 			for (const decode_plan& d : plan)
 			{
 				const launch_geometry g =
-					d.tiled ? launch_geometry{0, d.nz, tiled_part_bytes(d, n_head, n_kv, head_dim)}
+					d.tiled ? launch_geometry{0, d.nz, d.split_bytes + tiled_part_bytes(d, n_head, n_kv, head_dim)}
 					        : geometry_of(d.n, pos0 + d.t0, n_seq, window, causal, n_head, n_kv, head_dim, d.sk);
 				if (g.part_bytes > src.bytes)
 					return fail(NNC_ERR_INVALID_ARGUMENT,

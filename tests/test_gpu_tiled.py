@@ -111,3 +111,90 @@ def test_tiled_noalloc_matches_attend_device(orc):
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
     want = orc.attend_layer(q, K, V, kv_bf16=False, rows=n_seq, pos0=pos0, n_seq=pos0 + n_tok, **kw)
     assert errors(a, want)[0] <= 1e-3
+
+
+# Both sides of the rule for the three-part bf16 products (512 rows per KV head
+# and 4000 in all; 128-row blocks, 32-key groups): the smallest batch that takes
+# them and one token less, ragged last blocks, one split and many, windows on
+# both sides, rings that have wrapped, spans that start mid-group.
+T3_CASES = (
+    # n_head, n_kv, head_dim, causal, window, n_seq, n_tok, ring
+    (4, 1, 256, True, 0, 1011, 1000, False),
+    (4, 1, 256, True, 0, 1010, 999, False),
+    (3, 1, 256, False, 512, 1400, 1400, False),
+    (3, 1, 256, False, 0, 1337, 1337, False),
+    (16, 8, 128, True, 0, 1333, 261, False),
+    (16, 8, 128, True, 300, 1500, 300, True),
+    (8, 2, 64, True, 0, 555, 501, False),
+    (32, 8, 64, False, 200, 150, 150, False),
+    (4, 4, 256, True, 700, 2600, 1003, True),
+)
+
+
+@pytest.mark.parametrize("c", T3_CASES, ids=lambda c: "-".join(map(str, c)))
+def test_f32_three_part_products(orc, c):
+    """Against the oracle to 2e-5: fp32 products and sums on both sides (the
+    scores' fp32 rounding at |s| up to ~30 log2 units, about 30 * 2^-23 = 4e-6
+    per weight, on outputs up to ~4); the no-alloc entry point runs the same
+    launches, bit for bit; a gate on top."""
+    n_head, n_kv, hd, causal, window, n_seq, n_tok, ring = c
+    cfg = synth.AttnConfig(61, "t3", n_head, n_kv, hd, 1, kv_bf16=False, window=window, swa_period=2, tol=1e-3)
+    rows = nh.kv_rows(4 * n_seq, window, n_tok) if ring else n_seq + 5
+    pos0 = n_seq - n_tok
+    K, V = synth.cache_buffer(cfg, 0, rows, n_seq)
+    q = synth.qk_rows(cfg, 0, 0, np.arange(pos0, n_seq), n_head)
+    kw = dict(window=window, causal=causal, n_head=n_head, n_kv=n_kv, head_dim=hd, scale=cfg.attn_scale)
+    say(f"case three-part {c}: rows {rows}")
+    gate = np.random.default_rng(1).standard_normal(q.shape).astype(np.float32)
+    with nh.KVCache([rows], [cfg.kv_dim], bf16=False) as kv:
+        kv.append(0, 0, K, V)
+        got = kv.attend(0, q, pos0=pos0, n_seq=n_seq, **kw)
+        gated = kv.attend(0, q, pos0=pos0, n_seq=n_seq, gate=gate, **kw)
+        qd, od = hip_rt.malloc(q.nbytes), hip_rt.malloc(q.nbytes)
+        try:
+            hip_rt.to_device(qd, q)
+            kv.attend_device_noalloc(0, qd, od, n_tok=n_tok, pos0=pos0, n_seq=n_seq, **kw)
+            kv.sync()
+            fixed = hip_rt.to_host(np.empty_like(got), od)
+        finally:
+            hip_rt.free(qd)
+            hip_rt.free(od)
+    want = orc.attend_layer(q, K, V, kv_bf16=False, rows=rows, pos0=pos0, n_seq=n_seq, **kw)
+    ea, er = errors(got, want)
+    say(f"  max-abs {ea:.3e} max-rel {er:.3e}")
+    assert ea <= 2e-5
+    assert np.array_equal(fixed.view(np.uint32), got.view(np.uint32))
+    assert np.abs(gated - got / (1 + np.exp(-gate.astype(np.float64)))).max() <= 2e-6
+
+
+def test_f32_three_part_products_in_a_graph(orc):
+    """Captured before its scratch has grown a long F32 batch with one split
+    runs the fp32 kernel; replays agree with each other and, to 2e-5, with the
+    eager call."""
+    n_head, n_kv, hd, n = 64, 16, 64, 700  # (176 row blocks of 64 and 16 KV heads: one split)
+    cfg = synth.AttnConfig(62, "t3 graph", n_head, n_kv, hd, 1, kv_bf16=False)
+    K, V = synth.cache_buffer(cfg, 0, n, n)
+    q = synth.qk_rows(cfg, 0, 0, np.arange(n), n_head)
+    kw = dict(n_tok=n, pos0=0, n_head=n_head, n_kv=n_kv, head_dim=hd, scale=cfg.attn_scale)
+    with nh.KVCache([n], [cfg.kv_dim], bf16=False) as kv:
+        kv.append(0, 0, K, V)
+        qd, od = hip_rt.malloc(q.nbytes), hip_rt.malloc(q.nbytes)
+        try:
+            hip_rt.to_device(qd, q)
+            say("case three-part under capture")
+            g = hip_rt.Graph(kv.stream, lambda: kv.attend_device(0, qd, od, **kw))
+            first = None
+            for _ in range(3):
+                hip_rt.to_device(od, np.zeros_like(q))
+                g.launch(kv.stream)
+                kv.sync()
+                got = hip_rt.to_host(np.empty_like(q), od)
+                first = got if first is None else first
+                assert np.array_equal(got, first)
+            g.close()
+            kv.attend_device(0, qd, od, **kw)
+            kv.sync()
+            assert np.abs(hip_rt.to_host(np.empty_like(q), od) - first).max() <= 2e-5
+        finally:
+            hip_rt.free(qd)
+            hip_rt.free(od)
