@@ -608,3 +608,20 @@ def test_hip_gemv_many_vectors_in_a_graph(orc):
     finally:
         for d in dev:
             hip_rt.free(d)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3])
+def test_group_array_packing(n):
+    """A group's array holds what a structure per matrix holds: every form of
+    its entries (tables left out, None, own strides, numbers out of range)."""
+    from libllmcpu_amd import nnc_hip as nh
+    full = [((1 << 40, 2 << 40, 3 << 40), 4 << 40, 48), ((5, 6), 7, 16, 64), ((1 << 63,), 9, 0xFFFFFFFF, 1 << 40)]
+    odd = [((None, None, None), None, 16), ((5, None), 7, 32), ((1,), -1, -2)]
+    for mats in (full[:n], odd[:n], full[3 - n:], odd[3 - n:]):
+        try:
+            want = bytes(nh._mat_array(mats))
+        except TypeError:
+            with pytest.raises(TypeError):
+                nh._packed_mats(mats)
+            continue
+        assert bytes(nh._packed_mats(mats)) == want
