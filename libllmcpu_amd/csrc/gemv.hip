@@ -1,26 +1,36 @@
 // The weight gemvs on either side of nnc's attention (reference
 // src/libnnc/nn_ops.h:95-180; model.cpp:1189-1210 picks one by tensor type):
-// Y[t][r] = sum_k W[r][k] X[t][k] for up to 16 activation vectors against one
-// pass over the weights, W in BF16, in the Q8_0 split layout (int8 q, one
-// BF16 scale per 32-column block) or the Q4_S split layout (nibble q, BF16
+// Y[t][r] = sum_k W[r][k] X[t][k], W in BF16, in the Q8_0 split layout (int8 q,
+// one BF16 scale per 32-column block) or the Q4_S split layout (nibble q, BF16
 // scale and bias per block; reference docs/design.md:141-193).
 //
-// MFMA formulation (v_mfma_f32_16x16x32_bf16): 16 weight rows x 16 tokens per
-// product, one 32-column block per k-step. A = the rows' weights of the block
-// as bf16, exact for BF16 and for the integer q of Q8_0 (|q| <= 127) and Q4_S
-// (0..15). B = X^T split into bf16 hi + lo (x ~= hi + lo to about 16 bits), so
-// the product against the exact A is near-fp32 and the accumulation fp32. A
-// quantised block's product starts from zero and is scaled into the row's sum
-// with the block's scale; Q4_S adds bias * (block sum of x) in a second sum.
-//
-// Grid: (row groups of kGemvRows = 128, K splits). A work-group of 8
-// wavefronts (two work-groups per CU) stages its K range of X^T (hi, lo, and
-// for Q4_S the block sums) in LDS once; each wavefront then streams the
-// weights of its own 16 rows block by block over the whole range, kAhead<F>
-// blocks of loads in flight (BF16: every block of its split, at most 16,
-// issued before X^T is staged). With one K split the rows go straight to Y; with
-// several, each split writes a partial and a second kernel adds the splits in
-// split order, so results are the same run to run.
+// One vector (gemv_vec_kernel): x in LDS, fp32 products on the VALU, a
+// wavefront per pair of rows. More than one: MFMA products
+// (v_mfma_f32_16x16x32_bf16), 16 weight rows x 16 vectors, one 32-column block
+// per k-step. A = the rows' weights of the block as bf16, exact for BF16 and
+// for the integer q of Q8_0 (|q| <= 127) and Q4_S (0..15). B = X^T split into
+// bf16 hi + lo (x ~= hi + lo to about 16 bits), so the product against the
+// exact A is near-fp32 and the accumulation fp32. A quantised block's product
+// starts from zero and is scaled into the row's sum with the block's scale;
+// Q4_S adds bias * (block sum of x) in a second sum. Three kernels:
+//   gemv_kernel        2 to 16 vectors of wide matrices (gemv_stages_x has the
+//                      line). Grid: (row groups of kGemvRows = 128, K splits).
+//                      A work-group of 8 wavefronts (two work-groups per CU)
+//                      stages its K range of X^T (hi, lo, and for Q4_S the
+//                      block sums) in LDS once; each wavefront then streams
+//                      the weights of its own 16 rows block by block over the
+//                      whole range, kAhead<F> blocks of loads in flight (BF16:
+//                      every block of its split, at most 16, issued before X^T
+//                      is staged). With one K split the rows go straight to Y;
+//                      with several, each split writes a partial and a second
+//                      kernel adds the splits in split order;
+//   gemv_batch_kernel  the other 2 to 16 vectors, and up to 64. X is put into
+//                      operand order once by gemv_stage_x_kernel; a work-group
+//                      takes a few row tiles, its wavefronts share the columns,
+//                      and their sums meet in LDS: no partials in memory;
+//   gemv_tile_kernel   more vectors than that: tiles of rows x vectors over all
+//                      the columns, W and X through LDS.
+// The sums' orders are fixed, so results are the same run to run.
 #include "device_common.h"
 #include "kernels.h"
 
@@ -987,6 +997,18 @@ namespace nnchip
 			static constexpr int CW = 64 * CPL; // columns per wavefront load
 		};
 
+		// Whether a row pair's last chunk is one item for both rows: when it is at
+		// most half full, an item being as much work whatever its lanes hold
+		// (Q4_S, 2560 columns: three items per pair instead of four; 19456 rows
+		// 17.1 -> 14.6 us with the byte masks of vec_dot). Only Q4_S, whose VALU
+		// work bounds it: Q8_0 was no faster with it (17.3 -> 17.7 us).
+		template <int F>
+		bool vec_joint(int cols)
+		{
+			constexpr int CW = vec_shape<F>::CW;
+			return F == kGemvQ4S && (cols - 1) % CW < CW / 2;
+		}
+
 		template <int F>
 		struct vec_item
 		{
@@ -1013,14 +1035,13 @@ namespace nnchip
 			return kVecLaneOrder<F> ? (cols + vec_shape<F>::CW - 1) / vec_shape<F>::CW * vec_shape<F>::CW : cols;
 		}
 
-		// The lane's dot product of one item (16 bytes of a row at columns
-		// c0 ..) with x in LDS.
+		// A lane's dot product of one item (16 bytes of a row at columns c0 ..,
+		// those of lane `lane` of a chunk) with x in LDS.
 		template <int F>
-		__device__ __forceinline__ float vec_dot(const vec_item<F>& it, int c0, const float* s_x, int cols)
+		__device__ __forceinline__ float vec_dot(const vec_item<F>& it, int c0, int lane, const float* s_x, int cols)
 		{
 			constexpr int CPL = vec_shape<F>::CPL;
 			if (c0 >= cols) return 0.0f;
-			const int lane = threadIdx.x & 63;
 			// columns c0 + 4 g .. + 3 at xq + GS g
 			constexpr int GS = kVecLaneOrder<F> ? 256 : 4;
 			const float* xq = kVecLaneOrder<F> ? s_x + (c0 - lane * CPL) + 4 * lane : s_x + c0;
@@ -1063,30 +1084,35 @@ namespace nnchip
 				{
 					const float4 xl = *reinterpret_cast<const float4*>(xq + GS * u); // columns 4 u ..
 					const float4 xh = *reinterpret_cast<const float4*>(xq + GS * (4 + u)); // columns 16 + 4 u ..
-					const uint32_t b = it.w[u];
-					d = fmaf(static_cast<float>(b & 0xfu), xl.x, d);
-					d = fmaf(static_cast<float>((b >> 8) & 0xfu), xl.y, d);
-					d = fmaf(static_cast<float>((b >> 16) & 0xfu), xl.z, d);
-					d = fmaf(static_cast<float>((b >> 24) & 0xfu), xl.w, d);
-					d = fmaf(static_cast<float>((b >> 4) & 0xfu), xh.x, d);
-					d = fmaf(static_cast<float>((b >> 12) & 0xfu), xh.y, d);
-					d = fmaf(static_cast<float>((b >> 20) & 0xfu), xh.z, d);
-					d = fmaf(static_cast<float>(b >> 28), xh.w, d);
+					// (a byte per nibble: 19 instructions for eight weights with the
+					// byte conversions, against 24 with a bit-field extract per
+					// nibble, into which the compiler folds the masks unless it
+					// cannot see them)
+					uint32_t lo = it.w[u] & 0x0f0f0f0fu, hi = (it.w[u] >> 4) & 0x0f0f0f0fu;
+					asm("" : "+v"(lo), "+v"(hi));
+					d = fmaf(static_cast<float>(lo & 0xffu), xl.x, d);
+					d = fmaf(static_cast<float>((lo >> 8) & 0xffu), xl.y, d);
+					d = fmaf(static_cast<float>((lo >> 16) & 0xffu), xl.z, d);
+					d = fmaf(static_cast<float>(lo >> 24), xl.w, d);
+					d = fmaf(static_cast<float>(hi & 0xffu), xh.x, d);
+					d = fmaf(static_cast<float>((hi >> 8) & 0xffu), xh.y, d);
+					d = fmaf(static_cast<float>((hi >> 16) & 0xffu), xh.z, d);
+					d = fmaf(static_cast<float>(hi >> 24), xh.w, d);
 				}
 				return fmaf(it.bi, s_x[vec_x_floats<F>(cols) + c0 / 32], it.sc * d);
 			}
 		}
 
-		// 16 bytes of row r of matrix m at columns c0 .. (lanes past the row's
-		// end re-read its last bytes; their sums are not used), with the
-		// block's scale and bias.
+		// 16 bytes of row r0 (second: r0 + 1) of matrix m at columns c0 ..
+		// (lanes past the row's end re-read its last bytes; their sums are not
+		// used), with the block's scale and bias.
 		template <int F>
-		__device__ __forceinline__ vec_item<F> vec_load(const gemv_mat& m, int r, int c0, int cols)
+		__device__ __forceinline__ vec_item<F> vec_load(const gemv_mat& m, int r0, int second, int c0, int cols)
 		{
 			constexpr int CPL = vec_shape<F>::CPL;
 			const int cc = min(c0, cols - CPL);
 			vec_item<F> it;
-			const size_t off = static_cast<size_t>(r) * cols + cc;
+			const size_t off = static_cast<size_t>(r0) * cols + (second ? cols : 0) + cc;
 			if constexpr (F == kGemvBf16)
 				it.w = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(m.w) + off);
 			else if constexpr (F == kGemvQ8_0)
@@ -1095,7 +1121,7 @@ namespace nnchip
 				it.w = *reinterpret_cast<const u32x4*>(static_cast<const uint8_t*>(m.w) + off / 2);
 			if constexpr (F != kGemvBf16)
 			{
-				const size_t si = static_cast<size_t>(r) * (cols / 32) + cc / 32;
+				const size_t si = static_cast<size_t>(r0) * (cols / 32) + (second ? cols / 32 : 0) + cc / 32;
 				it.sc = bf16_bits_to_f32(m.scales[si]);
 				if constexpr (F == kGemvQ4S) it.bi = bf16_bits_to_f32(m.biases[si]);
 			}
@@ -1151,7 +1177,8 @@ namespace nnchip
 
 		// ARGMAX (BF16 only): no y; each wavefront keeps its best row and the
 		// work-group writes its best (value, row) to p.best[blockIdx.x].
-		template <int F, bool ARGMAX = false>
+		// JOINT: vec_joint.
+		template <int F, bool ARGMAX = false, bool JOINT = false>
 		__global__ __launch_bounds__(256) void gemv_vec_kernel(const gemv_params p)
 		{
 			static_assert(!ARGMAX || F == kGemvBf16, "argmax of a BF16 gemv only");
@@ -1162,12 +1189,14 @@ namespace nnchip
 			const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
 			// Items: for each of this wavefront's row pairs, chunk c of row 0,
-			// then of row 1, for every chunk c of CW columns. Two cursors walk
+			// then of row 1, for every chunk c of CW columns; where the last
+			// chunk is at most half full (JOINT), one item for both rows, row
+			// 1's in the upper half of the lanes. Two cursors walk
 			// them, the loads' (kVecAhead<F> ahead) and the sums': (pair, item within
 			// the pair), stepped by one item at a time (no division per item);
 			// a pair's matrix is looked up when the load cursor enters it.
 			const int nch = (p.cols + CW - 1) / CW;
-			const int per_pair = 2 * nch;
+			const int per_pair = 2 * nch - JOINT;
 			const int gw = blockIdx.x * 4 + wave, n_gw = gridDim.x * 4;
 			const int n_pairs = (p.rows + 1) / 2;
 			const int my_pairs = gw < n_pairs ? (n_pairs - 1 - gw) / n_gw + 1 : 0;
@@ -1191,7 +1220,14 @@ namespace nnchip
 			{
 				const bool past = l_pi >= my_pairs;
 				const int rem = past ? per_pair - 1 : l_rem;
-				const vec_item<F> it = vec_load<F>(l_m, l_r0 + ((rem & 1) & l_two), (rem >> 1) * CW + lane * CPL, p.cols);
+				const bool both = JOINT && rem == per_pair - 1;
+				const int sub = both ? lane & 31 : lane;
+				const int row = both ? lane >> 5 : rem & 1;
+				// (where an item holds one row its index stays scalar: as a lane's
+				// selection Q8_0 took 18.5 us for 19456 x 2560 instead of 17.3)
+				const vec_item<F> it = JOINT
+					? vec_load<F>(l_m, l_r0, row & l_two, (rem >> 1) * CW + sub * CPL, p.cols)
+					: vec_load<F>(l_m, l_r0 + ((rem & 1) & l_two), 0, (rem >> 1) * CW + lane * CPL, p.cols);
 				if (!past && ++l_rem == per_pair)
 				{
 					l_rem = 0;
@@ -1199,10 +1235,6 @@ namespace nnchip
 					if (l_pi < my_pairs) enter_pair();
 				}
 				return it;
-			};
-			auto dot = [&](const vec_item<F>& it, int c0) __attribute__((always_inline)) -> float
-			{
-				return vec_dot<F>(it, c0, s_x, p.cols);
 			};
 
 			// The first loads go out before x is staged.
@@ -1227,7 +1259,17 @@ namespace nnchip
 					ring[j] = load(); // past the end: a repeat, never under a branch
 					if (k < n_items) // uniform
 					{
-						acc[j & 1] += dot(it, (u_rem >> 1) * CW + lane * CPL);
+						if constexpr (JOINT)
+						{
+							const bool both = u_rem == per_pair - 1;
+							const int sub = both ? lane & 31 : lane;
+							const float d = vec_dot<F>(it, (u_rem >> 1) * CW + sub * CPL, sub, s_x, p.cols);
+							const bool second = both ? lane > 31 : (u_rem & 1) != 0;
+							acc[0] += second ? 0.0f : d;
+							acc[1] += second ? d : 0.0f;
+						}
+						else
+							acc[j & 1] += vec_dot<F>(it, (u_rem >> 1) * CW + lane * CPL, lane, s_x, p.cols);
 						if (u_rem == per_pair - 1) // the pair's last item: both rows are complete
 						{
 							const float y0 = wave_sum_dpp(acc[0]), y1 = wave_sum_dpp(acc[1]);
@@ -1509,7 +1551,12 @@ namespace nnchip
 			{
 			case kGemvBf16: gemv_vec_kernel<kGemvBf16><<<grid, 256, lds, stream>>>(p); return true;
 			case kGemvQ8_0: gemv_vec_kernel<kGemvQ8_0><<<grid, 256, lds, stream>>>(p); return true;
-			case kGemvQ4S: gemv_vec_kernel<kGemvQ4S><<<grid, 256, lds, stream>>>(p); return true;
+			case kGemvQ4S:
+				if (vec_joint<kGemvQ4S>(p.cols))
+					gemv_vec_kernel<kGemvQ4S, false, true><<<grid, 256, lds, stream>>>(p);
+				else
+					gemv_vec_kernel<kGemvQ4S><<<grid, 256, lds, stream>>>(p);
+				return true;
 			default: return false;
 			}
 		}

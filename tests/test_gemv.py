@@ -625,3 +625,22 @@ def test_group_array_packing(n):
                 nh._packed_mats(mats)
             continue
         assert bytes(nh._packed_mats(mats)) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [32, 1024, 1056, 2048, 2080, 3072, 3104, 5120])
+def test_hip_gemv_one_vector_row_ends(orc, cols):
+    """One vector at both sides of the joint last item (Q4_S, a last chunk of
+    2048 columns at most half full), row counts with and without a second row
+    in the last pair, against the oracle within the format's bound."""
+    import libllmcpu_amd as nh
+
+    for rows in (1, 37, 64):
+        rng = np.random.default_rng(cols + rows)
+        wf = (rng.standard_normal((rows, cols)) * 0.05).astype(np.float32)
+        x = (rng.standard_normal((1, cols)) * 2).astype(np.float32)
+        with nh.KVCache([16], [64]) as kv:
+            for fmt, wl in layouts(orc, wf).items():
+                print(f"case gemv row ends {fmt} {rows} x {cols}", flush=True)
+                got = kv.gemv(fmt, wl, x, rows=rows, cols=cols)
+                assert np.all(np.abs(got.astype(np.float64) - oracle_gemv(orc, fmt, wl, x)) <= bound(fmt, wl, x)), (fmt, rows)
