@@ -397,7 +397,7 @@ def gemv_bench(nh, hip_rt, kv, stream, timed) -> dict:
     return {"what": "Qwen3-4B layer weight gemvs (q, k, v, o, gate, up, down) per weight layout; n1 = one "
                     "vector (decode), n16 = a 16-token session batch; weights in HBM, rotated past the "
                     "Infinity Cache; four launches per layer (q/k/v and gate/up as nnc_hip_gemv_group calls)", "bound": "hbm", "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "kernels": "gemv_vec_kernel (one vector), gemv_kernel + gemv_reduce_kernel (batches)", **res}
+            "kernels": "gemv_vec_kernel (one vector), gemv_batch_kernel or gemv_kernel + gemv_reduce_kernel (batches)", **res}
 
 
 def decode_layer_bytes(span: int, n_kv: int, hd: int, n_head: int, esize: int) -> int:

@@ -206,7 +206,7 @@ nnc_status nnc_hip_kv_read(nnc_hip_kv* kv, int32_t buf, int32_t row0, int32_t n_
  * bits of its one-token call (the decode == batch property of reference
  * tests.cpp:2631-2661 that MTP verification relies on). Larger batches run
  * the MFMA prefill kernel (BF16, head_dim 64, 128 or 256 with a group of 1,
- * 2, 4 or 8) or the tiled fp32-MFMA kernel (F32, and the other head shapes
+ * 2, 4 or 8) or the tiled kernels (fp32 products; F32, and the other head shapes
  * with head_dim a multiple of 16), within tolerance, not bit-identical;
  * other shapes stay on the split-K kernels. Supported shapes: every even
  * head_dim up to 512 (as nnc, reference model.cpp:714) with a group
@@ -306,9 +306,9 @@ nnc_status nnc_hip_gemv_q4_s(nnc_hip_kv* kv, const uint8_t* qs, const uint16_t* 
  * kernels, the same sums per row). format is NNC_HIP_GEMV_BF16, _Q8_0 or
  * _Q4_S, n_mat 1 .. NNC_HIP_GEMV_MAX_GROUP, every matrix of cols columns in
  * that layout (scales for Q8_0 and Q4_S, biases for Q4_S, NULL otherwise);
- * XSUM as for nnc_hip_gemv_q4_s (ignored for other formats). One launch per
- * 16 vectors for the whole group when every matrix but the last has a
- * multiple of 16 rows (nnc's projections do), else one per matrix. Errors as
+ * XSUM as for nnc_hip_gemv_q4_s (ignored for other formats). The whole
+ * group runs as one product per 1024 vectors when every matrix but the last has a multiple of 16 rows (nnc's
+ * projections do), else each matrix by itself. Errors as
  * for the single-matrix calls, and NNC_ERR_INVALID_ARGUMENT for an unknown
  * format or n_mat out of range. */
 enum
