@@ -373,22 +373,30 @@ namespace nnchip
 		// group's K and V have one LDS buffer each: the next K loads (LDS-DMA)
 		// during this group's P . V, the next V during the next scores. us, one
 		// stream / three at once, tiled_kernel -> this: six layers of a 2048-token
-		// embedding call (five windowed) 408 / 318 -> 340 / 220, four of 1000
+		// embedding call (five windowed) 408 / 318 -> 345 / 222, four of 1000
 		// causal tokens of 4 x 256 244 / 171 -> 197 / 123, two of 300 tokens over
 		// 1500 keys of 16 x 128 133 / 90 -> 119 / 63. Bound by the matrix cores,
 		// and in a windowed layer (four groups per work-group) by Q's staging,
 		// the operands' kernel and the merge around them.
 		constexpr int kT3Block = kTiled3Block, kT3Keys = kTiled3Keys;
 
+		// x as bf16 parts, x = out[0] + out[1] + out[2] to 24 bits. ANY (K, V and
+		// Q; the weights are at most 2^8): a part holds at most the largest finite
+		// bf16, so a finite x near the fp32 limit stays finite, an infinite one is
+		// (largest, largest, inf), whose products with an operand are infinite of
+		// the right sign or finite, and NaN stays in the last part.
+		template <bool ANY>
 		__device__ __forceinline__ void split3(const float (&x)[8], u32x4 (&out)[3])
 		{
+			const float big = __uint_as_float(0x7f7f0000u);
+			auto lim = [&](float v) __attribute__((always_inline)) { return ANY ? fminf(fmaxf(v, -big), big) : v; };
 #pragma unroll
 			for (int j = 0; j < 4; ++j)
 			{
 				const float a = x[2 * j], b = x[2 * j + 1];
-				const uint32_t h = cvt_pk_bf16(a, b);
+				const uint32_t h = cvt_pk_bf16(lim(a), lim(b));
 				const float a1 = a - bf16_lo(h), b1 = b - bf16_hi(h);
-				const uint32_t m = cvt_pk_bf16(a1, b1);
+				const uint32_t m = cvt_pk_bf16(lim(a1), lim(b1));
 				out[0][j] = h;
 				out[1][j] = m;
 				out[2][j] = cvt_pk_bf16(a1 - bf16_lo(m), b1 - bf16_hi(m));
@@ -426,7 +434,7 @@ namespace nnchip
 					}
 					x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
 					x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
-					split3(x, o);
+					split3<true>(x, o);
 #pragma unroll
 					for (int c = 0; c < 3; ++c) *reinterpret_cast<u32x4*>(dst + (f * 3 + c) * 1024 + 16 * lane) = o[c];
 				}
@@ -437,7 +445,7 @@ namespace nnchip
 						const int k = key0 + 16 * (j >> 2) + 4 * g + (j & 3);
 						x[j] = k >= k_lo && k <= k_hi ? V[row(k) + 16 * f + r] : 0.0f;
 					}
-					split3(x, o);
+					split3<true>(x, o);
 #pragma unroll
 					for (int c = 0; c < 3; ++c)
 						*reinterpret_cast<u32x4*>(dst + kT3Bytes<HD> + (f * 3 + c) * 1024 + 16 * lane) = o[c];
@@ -549,7 +557,7 @@ namespace nnchip
 					const float4 v = *reinterpret_cast<const float4*>(p.q + qo[a] + 32 * kk + 8 * c + 4);
 					const float x[8] = {u.x * p.qscale, u.y * p.qscale, u.z * p.qscale, u.w * p.qscale,
 					                    v.x * p.qscale, v.y * p.qscale, v.z * p.qscale, v.w * p.qscale};
-					split3(x, q[kk][a]);
+					split3<true>(x, q[kk][a]);
 				}
 			}
 
@@ -636,7 +644,7 @@ namespace nnchip
 						ls += w[j];
 					}
 					l_run[a] += row4_sum(ls);
-					split3(w, pw[a]);
+					split3<false>(w, pw[a]);
 				}
 
 				t3_wait_barrier<ND>(); // V has landed; the next K may be in flight

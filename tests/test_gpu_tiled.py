@@ -198,3 +198,33 @@ def test_f32_three_part_products_in_a_graph(orc):
         finally:
             hip_rt.free(qd)
             hip_rt.free(od)
+
+
+def test_f32_three_part_special_values():
+    """Infinities, NaN and large values in K and V, every key attended: the same classes (finite, +inf, -inf, NaN) per element as shorter
+    batches of the same tokens, which run fp32 products, and the finite ones
+    within 2e-5 of theirs."""
+    n_head, n_kv, hd, n = 4, 1, 256, 1024
+    cfg = synth.AttnConfig(63, "t3 special", n_head, n_kv, hd, 1, kv_bf16=False)
+    K, V = synth.cache_buffer(cfg, 0, n, n)
+    K, V = K.copy(), V.copy()
+    V[17, 3], V[400, 4], V[900, 5] = np.inf, -np.inf, np.nan
+    # (a weight reaches 2^8 against its row's offset, and up to 1024 of them are
+    # summed before the division: both kernels are finite up to the limit / 2^18)
+    V[33, 6], V[33, 7] = np.finfo(np.float32).max / 2**18, -np.finfo(np.float32).max / 2**18
+    q = synth.qk_rows(cfg, 0, 0, np.arange(n), n_head)
+    q.reshape(n, n_head, hd)[:, :, 9] = np.abs(q.reshape(n, n_head, hd)[:, :, 9]) + 0.1
+    K[55, 9] = -np.inf  # (weight 0 in every row)
+    kw = dict(n_seq=n, causal=False, n_head=n_head, n_kv=n_kv, head_dim=hd, scale=cfg.attn_scale)
+    say("case three-part special values")
+    with nh.KVCache([n], [cfg.kv_dim], bf16=False) as kv:
+        kv.append(0, 0, K, V)
+        got = kv.attend(0, q, pos0=0, **kw)
+        want = np.concatenate([kv.attend(0, q[i:i + 256], pos0=i, **kw) for i in range(0, n, 256)])
+    for cls in (np.isfinite, np.isposinf, np.isneginf, np.isnan):
+        say(f"  {cls.__name__}: columns that differ {np.unique(np.argwhere(cls(got) != cls(want))[:, 1] % hd)}")
+        assert np.array_equal(cls(got), cls(want)), cls.__name__
+    assert np.isposinf(want).any() and np.isnan(want).any()
+    ok = np.isfinite(want)
+    g, w = got[ok].astype(np.float64), want[ok].astype(np.float64)
+    assert (np.abs(g - w) <= 2e-5 * (1 + np.abs(w))).all()
