@@ -434,6 +434,12 @@ namespace nnchip
 		{
 			return static_cast<u32x4*>(p.xs) + (static_cast<size_t>(blk) * p.x_tiles + tile) * 128;
 		}
+		// A descriptor of the staged X from block blk on, to its end (at most
+		// kGemvStagedMax bytes).
+		__device__ __forceinline__ __amdgpu_buffer_rsrc_t x_from(const gemv_params& p, int blk)
+		{
+			return __builtin_amdgcn_make_buffer_rsrc(x_staged(p, blk, 0), 0, (p.cols / 32 - blk) * p.x_tiles * 2048, 0x00020000);
+		}
 		__device__ __forceinline__ uint16_t* x_sums(const gemv_params& p, int step, int tile)
 		{
 			const size_t n = static_cast<size_t>(p.cols / 32) * p.x_tiles;
@@ -624,8 +630,8 @@ namespace nnchip
 		}
 
 		constexpr int kBatchWaves = 8;
-		// Y[t][r] for 16 RT rows per work-group and up to 16 TT vectors, W
-		// streamed once. The wavefronts split the columns (contiguous runs of
+		// Y[t][r] for 16 RT rows per work-group and TT = p.x_tiles tiles of 16
+		// vectors (every tile that is read is staged), W streamed once. The wavefronts split the columns (contiguous runs of
 		// whole pieces, the same whatever RT and the number of rows, so a row
 		// gets the same bits in any group) and run without a barrier until
 		// their sums meet in LDS, added in wavefront order: no K splits over
@@ -655,8 +661,7 @@ namespace nnchip
 			u32x4 xh[PB][TT], xl[PB][TT];
 			uint32_t scale[RT];
 			const uint32_t xs_block = static_cast<uint32_t>(p.x_tiles) * 2048u;
-			const __amdgpu_buffer_rsrc_t rx =
-				__builtin_amdgcn_make_buffer_rsrc(x_staged(p, min(i_lo * PB, nb - 1), 0), 0, 0x7fffffff, 0x00020000);
+			const __amdgpu_buffer_rsrc_t rx = x_from(p, min(i_lo * PB, nb - 1));
 			auto load = [&](int i) __attribute__((always_inline))
 			{
 #pragma unroll
@@ -825,8 +830,7 @@ namespace nnchip
 			const int b_lo = kg * h, p_hi = min(np, (kg + 1) * (h / PB));
 
 			const uint32_t xs_block = static_cast<uint32_t>(p.x_tiles) * 2048u;
-			const __amdgpu_buffer_rsrc_t rx =
-				__builtin_amdgcn_make_buffer_rsrc(x_staged(p, min(b_lo, nb - 1), 0), 0, 0x7fffffff, 0x00020000);
+			const __amdgpu_buffer_rsrc_t rx = x_from(p, min(b_lo, nb - 1));
 			unsigned char* const s_x = s_raw + kg * SLOTS * S::kSlot;
 			unsigned char* const s_w = s_raw + S::kLdsX + wave * NPW * RT * 1024; // [NPW][RT] pieces of this wavefront
 			uint32_t x_off[S::DX]; // DMA u: 1 KB (hi or lo of a tile) to its place [tile][hi, lo] in the slot
@@ -1426,9 +1430,12 @@ namespace nnchip
 			}
 		}
 
-		template <int F, int RT, int TT>
+		// p.x_tiles tiles of vectors: 1 to 4.
+		template <int F, int RT, int TT = 1>
 		void launch_batch(const gemv_params& p, hipStream_t stream)
 		{
+			if constexpr (TT < 4)
+				if (p.x_tiles != TT) return launch_batch<F, RT, TT + 1>(p, stream);
 			gemv_batch_kernel<F, RT, TT><<<(p.rows + 16 * RT - 1) / (16 * RT), 64 * kBatchWaves,
 			                               kBatchWaves * RT * TT * 1024, stream>>>(p);
 		}
@@ -1453,13 +1460,7 @@ namespace nnchip
 			{
 				// Two 16-row tiles per work-group halve the reads of X; one
 				// fills more CUs (from 160 work-groups on, two).
-				const bool two = p.rows >= 32 * 160;
-				if (p.n_batch <= 16)
-					two ? launch_batch<F, 2, 1>(p, stream) : launch_batch<F, 1, 1>(p, stream);
-				else if (p.n_batch <= 32)
-					two ? launch_batch<F, 2, 2>(p, stream) : launch_batch<F, 1, 2>(p, stream);
-				else
-					two ? launch_batch<F, 2, 4>(p, stream) : launch_batch<F, 1, 4>(p, stream);
+				p.rows >= 32 * 160 ? launch_batch<F, 2>(p, stream) : launch_batch<F, 1>(p, stream);
 				return;
 			}
 			// rows x vectors per work-group, by what fills the 256 CUs (us, BF16 /

@@ -518,6 +518,7 @@ def test_hip_gemv_argmax_row0_nan(orc, rows):
 # of 32-column blocks, fewer blocks than a loop pass, a last chunk of 1 and of 6.
 WIDE_SHAPES = [
     (33, 32, 17), (1000, 96, 32), (5136, 160, 33), (5136, 416, 64), (72, 2560, 20),
+    (72, 2560, 48), (1000, 96, 41), (5136, 1056, 48),
     (40, 64, 65), (129, 1056, 70), (4112, 672, 100), (9000, 352, 129), (16400, 96, 200), (2000, 224, 1030), (16, 32, 1025),
 ]
 

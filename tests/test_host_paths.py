@@ -1,0 +1,112 @@
+"""What the bridge's host code launches, without a GPU: the library over a HIP
+runtime of the test's own (hip_stub.cpp) that records launches and allocations.
+Each check runs in a process of its own, since a process binds one runtime."""
+from __future__ import annotations
+
+import ctypes as C
+import re
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve()
+CHECKS = {}
+
+
+def check(fn):
+    CHECKS[fn.__name__] = fn
+    return fn
+
+
+@pytest.fixture(scope="session")
+def stub(tmp_path_factory):
+    so = tmp_path_factory.mktemp("hip_stub") / "libhip_stub.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    f"-DNNC_STUB_SYMBOL_BYTES={32 << 20}", str(HERE.parent / "hip_stub.cpp"), "-o", str(so)], check=True)
+    return so
+
+
+class Runtime:
+    def __init__(self, so: str):
+        self.lib = C.CDLL(so, mode=C.RTLD_GLOBAL)  # before libnnc_hip.so is loaded
+        self.lib.stub_name.restype = C.c_char_p
+        self.lib.stub_pointer.restype = C.c_void_p
+        self.lib.stub_bytes_left.restype = C.c_size_t
+        self.lib.stub_bytes_left.argtypes = [C.c_void_p]
+        self.lib.stub_live.restype = C.c_size_t
+
+    def launches(self):
+        """(name, gemv fields, captured) of the launches since the last call of clear()."""
+        got = []
+        for i in range(self.lib.stub_launches()):
+            v = (C.c_int * 5)()
+            self.lib.stub_gemv(i, v)
+            got.append(dict(zip(("n_batch", "cols", "rows", "x_tiles", "n_split"), v), name=self.lib.stub_name(i).decode(),
+                            captured=bool(self.lib.stub_captured(i)), xs=self.lib.stub_pointer(i, 0),
+                            part=self.lib.stub_pointer(i, 1), split=self.lib.stub_pointer(i, 2)))
+        return got
+
+    def clear(self):
+        self.lib.stub_clear()
+
+    def left(self, p):
+        return self.lib.stub_bytes_left(p)
+
+    def capture(self, fn):
+        self.lib.stub_capture(1)
+        try:
+            fn()
+        finally:
+            self.lib.stub_capture(0)
+        assert not self.lib.stub_capture_invalid(), "a call that a capture does not allow"
+
+
+FORMATS = ("bf16", "q8_0", "q4_s")
+
+
+def gemv(kv, fmt, n, rows, cols):
+    """(addresses are not read: nothing runs)"""
+    kv.gemv_device(fmt, (1 << 20, 2 << 20, 3 << 20), 4 << 20, 5 << 20, rows=rows, cols=cols, n_batch=n)
+
+
+@check
+def staged_x_stays_in_its_allocation(rt, nh):
+    """Every 16-vector tile that a gemv kernel reads is one that was staged (the
+    kernel of up to 64 vectors reads as many as its instance has; the tile
+    kernel clamps), and the staged X fits its allocation, for every number of
+    vectors up to 64 and some above."""
+    for fmt in FORMATS:
+        for cols in (32, 512, 2048, 2560):
+            for rows in (16, 1000, 5136):
+                for n in (*range(2, 66), 80, 129, 1024):
+                    with nh.KVCache([16], [64]) as kv:
+                        rt.clear()
+                        gemv(kv, fmt, n, rows, cols)
+                        for l in rt.launches():
+                            if not l["xs"]:
+                                continue
+                            what = (fmt, cols, rows, n, l["name"])
+                            assert l["x_tiles"] == (n + 15) // 16, what
+                            nb = cols // 32
+                            need = l["x_tiles"] * (nb * 2048 + ((nb + 31) // 32 * 3072 if fmt == "q4_s" else 0))
+                            assert need <= rt.left(l["xs"]), what
+                            m = re.search(r"gemv_batch_kernelILi\d+ELi\d+ELi(\d+)E", l["name"])
+                            if m:
+                                assert int(m[1]) <= l["x_tiles"], what
+
+
+@pytest.mark.parametrize("name", sorted(CHECKS))
+def test_host_path(stub, name):
+    r = subprocess.run([sys.executable, str(HERE), str(stub), name], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+
+
+if __name__ == "__main__":
+    rt = Runtime(sys.argv[1])
+    sys.path.insert(0, str(HERE.parents[1]))
+    import libllmcpu_amd
+
+    libllmcpu_amd.set_log_callback(lambda level, msg: None)
+    CHECKS[sys.argv[2]](rt, libllmcpu_amd)
