@@ -230,15 +230,17 @@ nnc_status nnc_hip_attend_device(nnc_hip_kv* kv, int32_t buf, const float* q, fl
                                  int32_t n_kv, int32_t head_dim, float scale);
 
 /* Bytes of the fixed per-device scratch of nnc_hip_attend_device_noalloc
- * (split partials of decode and of tiled batches). */
+ * (split partials of decode and of tiled batches, and the K and V operands of
+ * long F32 batches). */
 #define NNC_HIP_NOALLOC_SCRATCH_BYTES (32u << 20)
 
 /* As nnc_hip_attend_device, for callers that cannot allocate device memory:
  * code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc. No counterpart in the reference. The call allocates nothing
  * (no hipMalloc, hipFree or allocating library routine): the split kernels'
- * partials go to a fixed array of NNC_HIP_NOALLOC_SCRATCH_BYTES in each
- * device's memory, which the library holds until the process ends. Every
+ * partials, and the K and V operands of a long F32 batch, go to a fixed array
+ * of NNC_HIP_NOALLOC_SCRATCH_BYTES in each device's memory, which the library
+ * holds until the process ends. Every
  * call on a GPU shares that GPU's array, and the calls are asynchronous: two
  * no-alloc calls on different caches of one GPU (each cache has its own
  * stream) overlap on the GPU and race on the array, even when one thread
@@ -355,7 +357,19 @@ nnc_status nnc_hip_argmax_f32(nnc_hip_kv* kv, const float* y, uint32_t n, int32_
 /* Waits for all work queued on the cache's stream. */
 nnc_status nnc_hip_kv_sync(nnc_hip_kv* kv);
 
-/* The cache's hipStream_t, for callers that order their own work on it. */
+/* The cache's hipStream_t, for callers that order their own work on it, or
+ * capture the device calls on it into a HIP graph. A captured call uses the
+ * cache's scratch as an eager one does. Nothing can be allocated during a
+ * capture: run the calls once before, or a call that needs more scratch than
+ * is there fails, or takes a way that needs none (a gemv of several vectors,
+ * and a long F32 batch with one split: same tolerance, other bits). Scratch
+ * that a later call outgrows is kept until the cache is freed (all that is
+ * kept so is shorter than what replaced it), so a graph may be replayed after
+ * calls of any size; its replays share the scratch with the cache's other
+ * calls and must be ordered with them (replay on this stream). A captured
+ * nnc_hip_kv_prep_append_device call reads the RoPE table that the cache
+ * holds at the replay, which is the last two calls', so it is not one to
+ * replay after calls at other positions. */
 void* nnc_hip_kv_stream(nnc_hip_kv* kv);
 
 /* Fills n elements at device address dst with N(0,1) values from the

@@ -190,6 +190,7 @@ struct nnc_hip_kv
 	unsigned* counts = nullptr; // kFuseCounts arrival counts of the fused decode merge (device, zero between calls)
 	dev_scratch rows_k;
 	dev_scratch rows_v;
+	std::vector<void*> retired; // outgrown scratch, which a captured graph may still use
 	host_staging pinned; // host rows in and out (q, gate, out; K/V appends; RoPE tables)
 	rope_table rope[2]; // the last two RoPE setups (Gemma 3 alternates local and global layers)
 	uint64_t rope_clock = 0;
@@ -211,22 +212,52 @@ namespace
 		for (dev_scratch* s : {&kv->part, &kv->q, &kv->gate, &kv->gemv_part, &kv->rows_k, &kv->rows_v,
 		                       &kv->rope[0].dev, &kv->rope[1].dev})
 			if (s->ptr) (void)hipFree(s->ptr);
+		for (void* ptr : kv->retired) (void)hipFree(ptr);
 		if (kv->pinned.ptr) (void)hipHostFree(kv->pinned.ptr);
 		if (kv->pinned.free) (void)hipEventDestroy(kv->pinned.free);
 		if (kv->stream) (void)hipStreamDestroy(kv->stream);
 		delete kv;
 	}
 
-	// Makes s at least `bytes` long; the old allocation is freed after the
-	// stream has drained.
+	// Whether the cache's stream is being captured into a graph (nothing can be
+	// allocated then).
+	bool capturing(const nnc_hip_kv* kv)
+	{
+		hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+		return hipStreamIsCapturing(kv->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+	}
+
+	// Makes s at least `bytes` long. The outgrown block stays allocated until
+	// the cache is freed: a graph captured from an earlier call goes on
+	// writing there when it is replayed. (Asking the stream on each call
+	// whether it is being captured, to keep only what a graph uses, took 0.2 us:
+	// 18 short decode calls 139 -> 143 us.) A block is at least twice as long as
+	// the one before it, so all outgrown ones together are shorter than the
+	// one in use; only where that does not fit is it just as long as needed.
 	nnc_status reserve(nnc_hip_kv* kv, dev_scratch& s, size_t bytes, const char* what)
 	{
 		if (s.bytes >= bytes) return NNC_OK;
 		NNC_HIP_TRY(hipStreamSynchronize(kv->stream), what);
-		if (s.ptr) NNC_HIP_TRY(hipFree(s.ptr), what);
+		if (s.ptr)
+		{
+			try
+			{
+				kv->retired.push_back(s.ptr);
+			}
+			catch (const std::bad_alloc&)
+			{
+				return fail(NNC_ERR_OUT_OF_MEMORY, "%s: out of host memory", what);
+			}
+		}
+		const size_t n = (std::max<size_t>(bytes, 256) + 255) & ~static_cast<size_t>(255), twice = 2 * s.bytes;
+		s = dev_scratch{};
+		if (twice > n && hipMalloc(&s.ptr, twice) == hipSuccess)
+		{
+			s.bytes = twice;
+			return NNC_OK;
+		}
+		(void)hipGetLastError(); // (the longer block's)
 		s.ptr = nullptr;
-		s.bytes = 0;
-		const size_t n = (std::max<size_t>(bytes, 256) + 255) & ~static_cast<size_t>(255);
 		NNC_HIP_TRY(hipMalloc(&s.ptr, n), what);
 		s.bytes = n;
 		return NNC_OK;
@@ -655,11 +686,7 @@ namespace
 					d.k_lo = k_lo;
 					d.k_hi = k_hi;
 					const size_t need = split + tiled_part_bytes(d, group * n_kv, n_kv, head_dim);
-					hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-					const bool there = src.ptr ? need <= src.bytes
-					                           : need <= kv->part.bytes ||
-					                                 (hipStreamIsCapturing(kv->stream, &st) == hipSuccess &&
-					                                  st == hipStreamCaptureStatusNone);
+					const bool there = src.ptr ? need <= src.bytes : need <= kv->part.bytes || !capturing(kv);
 					if (need <= kTiled3Scratch && there)
 					{
 						plan.push_back(d);
@@ -1153,11 +1180,9 @@ namespace
 		if (n_batch == 1) return 1;
 		const int nb = static_cast<int>(std::min<uint32_t>(n_batch, nnchip::kGemvWideBatch));
 		if (nnchip::gemv_staged_bytes(cols, nb, format) > nnchip::kGemvStagedMax) return nnchip::kGemvMaxBatch;
-		if (gemv_scratch_bytes(rows, cols, nb, format) > kv->gemv_part.bytes && nnchip::gemv_vec_fits(cols, 1, format))
-		{
-			hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-			if (hipStreamIsCapturing(kv->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone) return 1;
-		}
+		if (gemv_scratch_bytes(rows, cols, nb, format) > kv->gemv_part.bytes && nnchip::gemv_vec_fits(cols, 1, format) &&
+		    capturing(kv))
+			return 1;
 		return nnchip::kGemvWideBatch;
 	}
 

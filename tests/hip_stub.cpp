@@ -17,7 +17,8 @@ namespace
 	{
 		std::string name;
 		dim3 grid;
-		nnchip::gemv_params gemv; // gemv kernels
+		nnchip::gemv_params gemv; // kernels that take them
+		nnchip::decode_params attn;
 		const char* split; // tiled3 kernels: the operands
 		bool captured;
 	};
@@ -53,13 +54,15 @@ int stub_launches() { return static_cast<int>(g_launches.size()); }
 void stub_clear() { g_launches.clear(); }
 const char* stub_name(int i) { return g_launches[i].name.c_str(); }
 int stub_captured(int i) { return g_launches[i].captured; }
-// The staged X (0), partial sums (1) or tiled3 operands (2) of launch i.
+// The staged X (0), a gemv's partial sums (1), the tiled3 operands (2) or the
+// attention partials (3) of launch i, null where it has none.
 const void* stub_pointer(int i, int what)
 {
 	const launch& l = g_launches[i];
 	if (what == 0) return l.gemv.xs;
-	if (what == 1) return l.gemv.part;
-	return l.split;
+	if (what == 1) return l.gemv.n_split > 1 ? l.gemv.part : nullptr;
+	if (what == 2) return l.split;
+	return l.attn.n_split > 1 ? l.attn.part : nullptr;
 }
 // n_batch, cols, rows, x_tiles, n_split of a gemv launch.
 void stub_gemv(int i, int* out)
@@ -77,7 +80,12 @@ size_t stub_bytes_left(const void* p)
 	--it;
 	return c < it->first + it->second ? static_cast<size_t>(it->first + it->second - c) : 0;
 }
-size_t stub_live() { return g_live.size(); }
+size_t stub_live_bytes()
+{
+	size_t n = 0;
+	for (const auto& a : g_live) n += a.second;
+	return n;
+}
 
 // ---- the runtime ----
 hipError_t hipMalloc(void** p, size_t n)
@@ -181,7 +189,8 @@ hipError_t hipLaunchKernel(const void* fn, dim3 grid, dim3, void** args, size_t,
 	l.name = g_names[fn];
 	l.grid = grid;
 	l.captured = g_capturing;
-	if (l.name.find("gemv") != std::string::npos) l.gemv = *static_cast<nnchip::gemv_params*>(args[0]);
+	if (l.name.find("gemv_params") != std::string::npos) l.gemv = *static_cast<nnchip::gemv_params*>(args[0]);
+	if (l.name.find("decode_params") != std::string::npos) l.attn = *static_cast<nnchip::decode_params*>(args[0]);
 	if (l.name.find("tiled3") != std::string::npos) l.split = *static_cast<const char**>(args[1]);
 	g_launches.push_back(l);
 	return hipSuccess;

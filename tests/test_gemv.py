@@ -611,6 +611,73 @@ def test_hip_gemv_many_vectors_in_a_graph(orc):
             hip_rt.free(d)
 
 
+@pytest.mark.gpu
+def test_graph_replays_after_its_scratch_is_outgrown(orc):
+    """Warm up, capture (gemvs with X staged and with K splits, and a decode
+    token over several splits), run larger calls that outgrow every scratch,
+    and allocate over what they gave back: replays give the eager bits, and
+    write nothing outside."""
+    import libllmcpu_amd as nh
+    from libllmcpu_amd import hip_rt, synth
+
+    rng = np.random.default_rng(8)
+    rows, n, n_seq, big = 96, 16, 600, 1024
+    cfg = synth.AttnConfig(64, "graph growth", 16, 8, 128, 1, kv_bf16=False)
+    K, V = synth.cache_buffer(cfg, 0, n_seq, n_seq)
+    q = synth.qk_rows(cfg, 0, 0, np.array([n_seq - 1]), 16)
+    w = {c: layouts(orc, (rng.standard_normal((rows, c)) * 0.05).astype(np.float32))["bf16"][0] for c in (512, 4096)}
+    x = {c: rng.standard_normal((big, c)).astype(np.float32) for c in w}
+    with nh.KVCache([n_seq], [cfg.kv_dim], bf16=False) as kv:
+        kv.append(0, 0, K, V)
+        dev = {}
+        try:
+            def put(name, a):
+                dev[name] = hip_rt.malloc(a.nbytes)
+                hip_rt.to_device(dev[name], np.ascontiguousarray(a))
+            for c in w:
+                put(f"w{c}", w[c])
+                put(f"x{c}", x[c])
+            put("y", np.zeros((2, big, rows), np.float32))
+            put("q", np.repeat(q, 16, 0))
+            put("o", np.zeros((16, q.size), np.float32))
+
+            def step():
+                for i, c in enumerate(w):
+                    kv.gemv_device("bf16", (dev[f"w{c}"],), dev[f"x{c}"], dev["y"] + 4 * i * big * rows, rows=rows, cols=c, n_batch=n)
+                kv.attend_device(0, dev["q"], dev["o"], n_tok=1, pos0=n_seq - 1, n_head=16, n_kv=8, head_dim=128, scale=0.1)
+
+            def outputs():
+                kv.sync()
+                y = hip_rt.to_host(np.empty((2, big, rows), np.float32), dev["y"])
+                return y[:, :n].copy(), hip_rt.to_host(np.empty_like(q), dev["o"])
+
+            print("case graph: warm up and capture", flush=True)
+            step()
+            want = outputs()
+            g = hip_rt.Graph(kv.stream, step)
+            print("case graph: larger calls", flush=True)
+            for c in w:
+                kv.gemv_device("bf16", (dev[f"w{c}"],), dev[f"x{c}"], dev["y"], rows=rows, cols=c, n_batch=big)
+            kv.attend_device(0, dev["q"], dev["o"], n_tok=16, pos0=n_seq - 16, n_head=16, n_kv=8, head_dim=128, scale=0.1)
+            kv.sync()
+            guard = np.full(1 << 20, 7, np.uint8)
+            for i in range(8):
+                put(f"guard{i}", guard)
+            for rep in range(3):
+                print(f"case graph: replay {rep}", flush=True)
+                hip_rt.to_device(dev["y"], np.zeros((2, big, rows), np.float32))
+                hip_rt.to_device(dev["o"], np.zeros_like(q))
+                g.launch(kv.stream)
+                got = outputs()
+                assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(got, want)), rep
+                for i in range(8):
+                    assert np.array_equal(hip_rt.to_host(np.empty_like(guard), dev[f"guard{i}"]), guard)
+            g.close()
+        finally:
+            for d in dev.values():
+                hip_rt.free(d)
+
+
 @pytest.mark.parametrize("n", [1, 2, 3])
 def test_group_array_packing(n):
     """A group's array holds what a structure per matrix holds: every form of

@@ -35,7 +35,7 @@ class Runtime:
         self.lib.stub_pointer.restype = C.c_void_p
         self.lib.stub_bytes_left.restype = C.c_size_t
         self.lib.stub_bytes_left.argtypes = [C.c_void_p]
-        self.lib.stub_live.restype = C.c_size_t
+        self.lib.stub_live_bytes.restype = C.c_size_t
 
     def launches(self):
         """(name, gemv fields, captured) of the launches since the last call of clear()."""
@@ -45,7 +45,7 @@ class Runtime:
             self.lib.stub_gemv(i, v)
             got.append(dict(zip(("n_batch", "cols", "rows", "x_tiles", "n_split"), v), name=self.lib.stub_name(i).decode(),
                             captured=bool(self.lib.stub_captured(i)), xs=self.lib.stub_pointer(i, 0),
-                            part=self.lib.stub_pointer(i, 1), split=self.lib.stub_pointer(i, 2)))
+                            scratch=[p for p in (self.lib.stub_pointer(i, w) for w in range(4)) if p]))
         return got
 
     def clear(self):
@@ -95,6 +95,45 @@ def staged_x_stays_in_its_allocation(rt, nh):
                             m = re.search(r"gemv_batch_kernelILi\d+ELi\d+ELi(\d+)E", l["name"])
                             if m:
                                 assert int(m[1]) <= l["x_tiles"], what
+
+
+def attend(kv, n_tok, pos0=0, *, n_head=8, n_kv=8, head_dim=64):
+    kv.attend_device(0, 1 << 20, 2 << 20, n_tok=n_tok, pos0=pos0, n_head=n_head, n_kv=n_kv, head_dim=head_dim, scale=0.1)
+
+
+@check
+def scratch_that_a_graph_uses_outlives_larger_calls(rt, nh):
+    """Warm up, capture, run a larger call: what the captured launches point to
+    is still allocated, and given back with the cache. What was outgrown over
+    many steps is together no longer than what is in use."""
+    rows, dim = 4096, 512
+    calls = {  # (BF16 cache, captured, larger)
+        "staged X": (True, lambda kv: gemv(kv, "bf16", 16, 1024, 512), lambda kv: gemv(kv, "bf16", 1024, 1024, 512)),
+        "K splits": (True, lambda kv: gemv(kv, "bf16", 16, 1024, 2560), lambda kv: gemv(kv, "bf16", 16, 8192, 2560)),
+        "decode": (False, lambda kv: attend(kv, 1, 300), lambda kv: attend(kv, 16, 4000)),
+        "long F32": (False, lambda kv: attend(kv, 1024), lambda kv: attend(kv, 2048)),
+    }
+    before = rt.lib.stub_live_bytes()
+    for name, (bf16, small, large) in calls.items():
+        with nh.KVCache([rows], [dim], bf16=bf16) as kv:
+            small(kv)
+            rt.clear()
+            rt.capture(lambda: small(kv))
+            held = {p for l in rt.launches() for p in l["scratch"]}
+            left = {p: rt.left(p) for p in held}
+            assert held and all(left.values()), name
+            rt.clear()
+            large(kv)
+            assert held.isdisjoint(p for l in rt.launches() for p in l["scratch"]), f"{name}: the scratch did not grow"
+            assert all(rt.left(p) == left[p] for p in held), name
+        assert rt.lib.stub_live_bytes() == before, name
+    with nh.KVCache([rows], [dim]) as kv:
+        empty = rt.lib.stub_live_bytes()
+        for n in range(2, 1025):
+            rt.clear()
+            gemv(kv, "bf16", n, 1024, 512)
+        in_use = rt.left(rt.launches()[0]["xs"])
+        assert in_use <= 2 * 1024 * 512 * 4 and rt.lib.stub_live_bytes() - empty < 2 * in_use
 
 
 @pytest.mark.parametrize("name", sorted(CHECKS))
