@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <cstdint>
 
 namespace nnchip
@@ -245,11 +246,6 @@ namespace nnchip
 		int mrow[kGemvMaxMats + 1];
 		const float* x; // [n_batch] vectors of cols floats, x_stride apart
 		const float* xsum; // Q4_S: [n_batch] runs of cols / 32 block sums, xsum_stride apart; or null
-		// X as matrix operands (gemv_staged_bytes; written by the launch's first
-		// kernel) where gemv_stages_x; null: the other kernels, which read x
-		// itself.
-		void* xs;
-		int x_tiles; // tiles of 16 vectors
 		float* part; // [n_split][n_batch][rows] partial sums when n_split > 1 (stacked rows)
 		size_t x_stride, xsum_stride;
 		int rows, cols, n_batch; // rows: all matrices' rows
@@ -259,7 +255,17 @@ namespace nnchip
 		float2* best; // [work-groups] (value, row as int bits; row -1 when none)
 		int* argmax; // the result, then whether y[0] is NaN
 		int first_sticks; // 1: the result is 0 when y[0] is NaN (the reference's linear scan from y[0])
+		int x_tiles; // tiles of 16 vectors in xs
+		// X as matrix operands (gemv_staged_bytes; written by the launch's first
+		// kernel) where gemv_stages_x; null: the other kernels, which read x
+		// itself.
+		void* xs;
 	};
+	// What the one-vector kernel reads before its first load lies in the first
+	// three 64-byte lines of the arguments: with rows and cols in a fourth it
+	// started 0.2 us later (640 x 1024 BF16 3.8 -> 4.0 us per launch of a graph,
+	// 2560 x 4096 9.0 -> 9.2).
+	static_assert(offsetof(gemv_params, cols) + sizeof(int) <= 192, "gemv_params' order");
 
 	// K splits of gemv_kernel.
 	void gemv_plan(int cols, int n_batch, int format, int& n_split, int& split_blocks);
