@@ -1430,14 +1430,18 @@ namespace nnchip
 			}
 		}
 
-		// p.x_tiles tiles of vectors: 1 to 4.
+		// p.x_tiles tiles of vectors: 1 to 4. (Q4_S with four: one row tile, since
+		// two spilled 61 registers: 64 vectors of 19456 x 2560 103 us, of 10240 x
+		// 9728 243; with one 63 and 110.)
 		template <int F, int RT, int TT = 1>
 		void launch_batch(const gemv_params& p, hipStream_t stream)
 		{
 			if constexpr (TT < 4)
 				if (p.x_tiles != TT) return launch_batch<F, RT, TT + 1>(p, stream);
-			gemv_batch_kernel<F, RT, TT><<<(p.rows + 16 * RT - 1) / (16 * RT), 64 * kBatchWaves,
-			                               kBatchWaves * RT * TT * 1024, stream>>>(p);
+			if constexpr (F == kGemvQ4S && RT == 2 && TT == 4) return launch_batch<F, 1, TT>(p, stream);
+			else
+				gemv_batch_kernel<F, RT, TT><<<(p.rows + 16 * RT - 1) / (16 * RT), 64 * kBatchWaves,
+				                               kBatchWaves * RT * TT * 1024, stream>>>(p);
 		}
 
 		template <int F, int RT, int TT, int WR, int SLOTS, int NPW>
