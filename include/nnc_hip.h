@@ -309,9 +309,10 @@ nnc_status nnc_hip_gemv_q4_s(nnc_hip_kv* kv, const uint8_t* qs, const uint16_t* 
  * _Q4_S, n_mat 1 .. NNC_HIP_GEMV_MAX_GROUP, every matrix of cols columns in
  * that layout (scales for Q8_0 and Q4_S, biases for Q4_S, NULL otherwise);
  * XSUM as for nnc_hip_gemv_q4_s (ignored for other formats). The whole
- * group runs as one product per 1024 vectors when every matrix but the last has a multiple of 16 rows (nnc's
- * projections do), else each matrix by itself. Errors as
- * for the single-matrix calls, and NNC_ERR_INVALID_ARGUMENT for an unknown
+ * group runs as one product (per 1024 vectors; fewer for few rows of many
+ * columns) when every matrix but the last has a multiple of 16 rows (nnc's
+ * projections do), else each matrix by itself. Errors as for the
+ * single-matrix calls, and NNC_ERR_INVALID_ARGUMENT for an unknown
  * format or n_mat out of range. */
 enum
 {

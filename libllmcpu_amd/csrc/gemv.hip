@@ -1460,7 +1460,7 @@ namespace nnchip
 		{
 			const int nb = p.cols / 32, items = (F == kGemvQ4S ? (nb + 31) & ~31 : nb) * p.x_tiles;
 			gemv_stage_x_kernel<F><<<(items + 3) / 4, 256, 0, stream>>>(p);
-			if (p.n_batch <= 64)
+			if (p.n_batch <= kGemvBatchMax)
 			{
 				// Two 16-row tiles per work-group halve the reads of X; one
 				// fills more CUs (from 160 work-groups on, two).
@@ -1517,6 +1517,37 @@ namespace nnchip
 	{
 		if (gemv_vec_fits(cols, n_batch, format)) return false;
 		return n_batch > kGemvMaxBatch || cols <= (format == kGemvBf16 ? 2048 : 6144);
+	}
+
+	// One launch takes all the vectors up to kGemvWideBatch, but where the kernel
+	// of that number leaves most of the chip idle: a work-group walks all the
+	// columns, so few rows of many columns are a long chain on few CUs. 65 and
+	// more vectors then run 64 at a time through gemv_batch_kernel, whose
+	// wavefronts share the columns, and 17 and more of the widest matrices 16 at
+	// a time through gemv_kernel, whose K splits give more work-groups. Graph
+	// replays of one stream, us, 16 at a time / 64 at a time / all in
+	// gemv_tile_kernel, 80 and 96 vectors: BF16 1024 x 9728 67 / 59 / 90 and 80 /
+	// 69 / 90, 2048 x 8192 67 / 53 / 77 and 81 / 59 / 77; Q8_0 1024 x 9728 69 /
+	// 58 / 108 and 82 / 72 / 108, 2560 x 9728 106 / 68 / 110 and 127 / 76 / 111;
+	// Q4_S 1024 x 7168 72 / 45 / 82 and 86 / 48 / 83. Three streams at once fill
+	// the CUs that one leaves idle: 64 at a time is then slower than all at once
+	// (BF16 2048 x 8192, 80 and 96 vectors, 32 / 28 and 37 / 30; quantised at 128
+	// vectors, 2560 x 9728 53 / 45), so the lines are where all at once is also
+	// slower than 16 at a time for one stream. 16 at a time / all at once: BF16
+	// 640 x 9728 26 / 30 (32 vectors), 640 x 14336 70 / 131 (80), Q8_0 1024 x
+	// 14336 33 / 43 (32). The rows are those of one matrix, and the matrices of a
+	// group that differ here run by themselves: a matrix gets the same bits
+	// alone and in a group.
+	int gemv_launch_vectors(int rows, int cols, int n_batch, int format)
+	{
+		const bool bf16 = format == kGemvBf16;
+		const int widest = bf16 ? 7680 : (format == kGemvQ8_0 ? 12288 : 16384);
+		if (gemv_staged_bytes(cols, std::min(n_batch, kGemvWideBatch), format) > kGemvStagedMax) return kGemvMaxBatch;
+		if (rows <= 1024 && n_batch > kGemvMaxBatch && n_batch <= (cols - widest) / 64) return kGemvMaxBatch;
+		if (rows <= (bf16 ? 2048 : 3072) && cols >= (bf16 ? 7168 : 6144) && n_batch > kGemvBatchMax &&
+		    n_batch <= (!bf16 ? 112 : (rows <= 1024 ? 96 : 80)))
+			return kGemvBatchMax;
+		return kGemvWideBatch;
 	}
 
 	size_t gemv_staged_bytes(int cols, int n_batch, int format)

@@ -197,9 +197,10 @@ namespace nnchip
 	// t < n_batch, W in one of nnc's three weight layouts.
 	constexpr int kGemvBf16 = 0, kGemvQ8_0 = 1, kGemvQ4S = 2;
 	constexpr int kGemvMaxBatch = 16; // vectors of one gemv_kernel launch
-	// Vectors of one launch with staged X (gemv_params::xs), and the bytes its
-	// staging may take (32-bit offsets).
-	constexpr int kGemvWideBatch = 1024;
+	// Vectors of one launch with staged X (gemv_params::xs), those of them that
+	// gemv_batch_kernel takes, and the bytes the staging may take (32-bit
+	// offsets).
+	constexpr int kGemvWideBatch = 1024, kGemvBatchMax = 64;
 	constexpr size_t kGemvStagedMax = size_t{1} << 30;
 	constexpr size_t kGemvLdsBudget = 64 << 10; // dynamic LDS per one-vector gemv work-group
 	// The batch kernel: weight rows per work-group (16 per wavefront) and its
@@ -274,6 +275,9 @@ namespace nnchip
 	// takes.
 	bool gemv_stages_x(int cols, int n_batch, int format);
 	size_t gemv_staged_bytes(int cols, int n_batch, int format);
+
+	// Most vectors per launch of a gemv of n_batch.
+	int gemv_launch_vectors(int rows, int cols, int n_batch, int format);
 
 	bool launch_gemv(const gemv_params& p, hipStream_t stream);
 

@@ -1172,24 +1172,23 @@ namespace
 		return n_split > 1 ? static_cast<size_t>(n_split) * nb * static_cast<size_t>(rows) * sizeof(float) : 0;
 	}
 
-	// Vectors per launch of a gemv of n_batch: all of them up to kGemvWideBatch;
-	// while the stream is captured into a graph and the scratch would have to
-	// grow (nothing can be allocated then), one, on the one-vector kernel.
-	static uint32_t gemv_chunk(const nnc_hip_kv* kv, int rows, int cols, uint32_t n_batch, int format)
+	// Vectors per launch of a gemv of n_batch, `most` by size; while the stream is
+	// captured into a graph and the scratch would have to grow (nothing can be
+	// allocated then), one, on the one-vector kernel.
+	static uint32_t gemv_chunk(const nnc_hip_kv* kv, int rows, int cols, uint32_t n_batch, int format, int most)
 	{
 		if (n_batch == 1) return 1;
-		const int nb = static_cast<int>(std::min<uint32_t>(n_batch, nnchip::kGemvWideBatch));
-		if (nnchip::gemv_staged_bytes(cols, nb, format) > nnchip::kGemvStagedMax) return nnchip::kGemvMaxBatch;
+		const int nb = static_cast<int>(std::min<uint32_t>(n_batch, most));
 		if (gemv_scratch_bytes(rows, cols, nb, format) > kv->gemv_part.bytes && nnchip::gemv_vec_fits(cols, 1, format) &&
 		    capturing(kv))
 			return 1;
-		return nnchip::kGemvWideBatch;
+		return most;
 	}
 
 	// Weight gemvs over the same X on the context's stream: one launch per
 	// chunk of gemv_chunk vectors for all the matrices together (stacked along
 	// the rows), or one per matrix when a matrix other than the last has a row
-	// count that is not a multiple of 16.
+	// count that is not a multiple of 16 or their rows ask for different chunks.
 	static nnc_status gemv_impl(nnc_hip_kv* kv, int format, int n_mat, const nnc_hip_gemv_mat* mats, const float* X,
 	                     size_t x_stride, const float* XSUM, size_t xsum_stride, uint32_t cols, uint32_t n_batch)
 	{
@@ -1223,6 +1222,14 @@ namespace
 			return fail(NNC_ERR_INVALID_ARGUMENT, "strides %zu / %zu for %u columns", x_stride, xsum_stride, cols);
 		if ((reinterpret_cast<uintptr_t>(X) & 15) || x_stride % 4 != 0)
 			return fail(NNC_ERR_INVALID_ARGUMENT, "X must be 16-byte aligned, x_stride a multiple of 4");
+		int most = 0;
+		for (int m = 0; m < n_mat; ++m)
+		{
+			const int v = nnchip::gemv_launch_vectors(static_cast<int>(mats[m].rows), static_cast<int>(cols),
+			                                          static_cast<int>(std::min<uint32_t>(n_batch, INT_MAX)), format);
+			if (m > 0 && v != most) stackable = false;
+			most = v;
+		}
 		if (!stackable)
 		{
 			for (int m = 0; m < n_mat; ++m)
@@ -1232,7 +1239,7 @@ namespace
 		}
 		uint32_t rows[nnchip::kGemvMaxMats];
 		for (int m = 0; m < n_mat; ++m) rows[m] = mats[m].rows;
-		const uint32_t chunk = gemv_chunk(kv, static_cast<int>(total), static_cast<int>(cols), n_batch, format);
+		const uint32_t chunk = gemv_chunk(kv, static_cast<int>(total), static_cast<int>(cols), n_batch, format, most);
 		for (uint32_t t0 = 0; t0 < n_batch; t0 += chunk)
 		{
 			const int nb = static_cast<int>(std::min<uint32_t>(n_batch - t0, chunk));

@@ -570,6 +570,48 @@ def test_hip_gemv_many_vectors(orc, rows, cols, n):
                         hip_rt.free(d)
 
 
+# Few rows of many columns: 64 vectors at a time (a rest of 1, 6 and 32), and 16
+# at a time (a rest of 1 and 16).
+FEW_ROWS = [(40, 7168, 65), (129, 9760, 70), (72, 7200, 96), (24, 8800, 17), (33, 9728, 32)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,n", FEW_ROWS, ids=[f"{r}x{c}x{n}" for r, c, n in FEW_ROWS])
+def test_hip_gemv_few_rows_of_many_columns(orc, rows, cols, n):
+    """To the bound of the smaller batches, every vector; and a group with a
+    matrix of more rows, which takes all the vectors at once, gives each
+    matrix the bits of its own call."""
+    import libllmcpu_amd as nh
+    from libllmcpu_amd import hip_rt
+
+    rng = np.random.default_rng(rows + cols + n)
+    rows2 = 3088
+    wf = (rng.standard_normal((rows2, cols)) * 0.05).astype(np.float32)
+    x = (rng.standard_normal((n, cols)) * 2).astype(np.float32)
+    r16 = rows // 16 * 16
+    with nh.KVCache([16], [64]) as kv:
+        for fmt, wl in layouts(orc, wf).items():
+            print(f"case gemv {fmt} {rows} x {cols}, {n} vectors", flush=True)
+            got = kv.gemv(fmt, tuple(np.ascontiguousarray(a[:rows]) for a in wl), x, rows=rows, cols=cols)
+            few = tuple(a[:rows] for a in wl)
+            assert np.all(np.abs(got.astype(np.float64) - oracle_gemv(orc, fmt, tuple(map(np.ascontiguousarray, few)), x))
+                          <= bound(fmt, few, x)), fmt
+            big = kv.gemv(fmt, wl, x, rows=rows2, cols=cols)
+            dev = [hip_rt.malloc(a.nbytes) for a in (*wl, x)] + [hip_rt.malloc(n * (r16 + rows2) * 4)]
+            try:
+                for d, a in zip(dev, (*wl, x)):
+                    hip_rt.to_device(d, a)
+                w, y = tuple(dev[:len(wl)]), dev[-1]
+                kv.gemv_group_device(fmt, [(w, y, r16), (w, y + 4 * n * r16, rows2)], dev[len(wl)], cols=cols, n_batch=n)
+                kv.sync()
+                both = hip_rt.to_host(np.empty(n * (r16 + rows2), np.float32), y)
+                assert np.array_equal(both[:n * r16].reshape(n, r16).view(np.uint32), np.ascontiguousarray(got[:, :r16]).view(np.uint32)), fmt
+                assert np.array_equal(both[n * r16:].reshape(n, rows2).view(np.uint32), big.view(np.uint32)), fmt
+            finally:
+                for d in dev:
+                    hip_rt.free(d)
+
+
 @pytest.mark.gpu
 def test_hip_gemv_many_vectors_in_a_graph(orc):
     """Captured by a cache whose scratch has not grown (nothing can be

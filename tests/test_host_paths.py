@@ -97,6 +97,45 @@ def staged_x_stays_in_its_allocation(rt, nh):
                                 assert int(m[1]) <= l["x_tiles"], what
 
 
+def route(launches):
+    """(kernel without its sizes, vectors, K splits) of each launch."""
+    return [(re.search(r"gemv_(?:[a-z]+_)*kernel", l["name"])[0], l["n_batch"], l["n_split"]) for l in launches]
+
+
+@check
+def many_vectors_of_few_wide_rows(rt, nh):
+    """Where a work-group per tile would leave the chip idle the vectors run 64 or
+    16 at a time; and a group's matrices go the way of their own calls."""
+    with nh.KVCache([16], [64]) as kv:
+        def launched(fmt, rows, cols, n):
+            rt.clear()
+            if isinstance(rows, int):
+                gemv(kv, fmt, n, rows, cols)
+            else:
+                kv.gemv_group_device(fmt, [((1 << 20, 2 << 20, 3 << 20)[:1 + FORMATS.index(fmt)], 5 << 20, r) for r in rows],
+                                     4 << 20, cols=cols, n_batch=n)
+            return route(l for l in rt.launches() if "stage_x" not in l["name"] and "reduce" not in l["name"])
+
+        for fmt in FORMATS:
+            for n in (65, 80, 96, 97, 112, 113):
+                got = launched(fmt, 1024, 9728, n)
+                if n <= (96 if fmt == "bf16" else 112):
+                    assert got[0][:2] == ("gemv_batch_kernel", 64) and sum(g[1] for g in got) == n, (fmt, n, got)
+                else:
+                    assert got == [("gemv_tile_kernel", n, 1)], (fmt, n, got)
+            assert launched(fmt, 8192, 9728, 80) == [("gemv_tile_kernel", 80, 1)]
+            assert launched(fmt, 1024, 2560, 80) == [("gemv_tile_kernel", 80, 1)]
+        assert [g[:2] for g in launched("bf16", 640, 9728, 32)] == [("gemv_kernel", 16)] * 2
+        for fmt in FORMATS:
+            for cols in (512, 2560, 6144, 9728, 16384):
+                for n in (2, 16, 17, 40, 64, 65, 100, 130, 1030):
+                    for rows in ((4096, 1024, 1024), (1024, 1024), (1040, 3072, 16)):
+                        alone = [launched(fmt, r, cols, n) for r in rows]
+                        group = launched(fmt, rows, cols, n)
+                        want = alone[0] if all(a == alone[0] for a in alone) else [x for a in alone for x in a]
+                        assert group == want, (fmt, cols, n, rows, group, alone)
+
+
 def attend(kv, n_tok, pos0=0, *, n_head=8, n_kv=8, head_dim=64):
     kv.attend_device(0, 1 << 20, 2 << 20, n_tok=n_tok, pos0=pos0, n_head=n_head, n_kv=n_kv, head_dim=head_dim, scale=0.1)
 
