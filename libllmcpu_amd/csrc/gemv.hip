@@ -13,8 +13,8 @@
 // exact A is near-fp32 and the accumulation fp32. A quantised block's product
 // starts from zero and is scaled into the row's sum with the block's scale;
 // Q4_S adds bias * (block sum of x) in a second sum. Three kernels:
-//   gemv_kernel        2 to 16 vectors of wide matrices (gemv_stages_x has the
-//                      line). Grid: (row groups of kGemvRows = 128, K splits).
+//   gemv_kernel        2 to 16 vectors of wide and of narrow matrices
+//                      (gemv_stages_x has the lines). Grid: (row groups of kGemvRows = 128, K splits).
 //                      A work-group of 8 wavefronts (two work-groups per CU)
 //                      stages its K range of X^T (hi, lo, and for Q4_S the
 //                      block sums) in LDS once; each wavefront then streams
@@ -1504,19 +1504,32 @@ namespace nnchip
 		split_blocks = (nb + n_split - 1) / n_split;
 	}
 
-	// Up to 16 vectors run either kernel. One stream / three at once, 16 vectors,
-	// us, gemv_kernel against gemv_batch_kernel (with its staging): Q8_0 6144 x
-	// 2560 16.4 / 10.1 against 12.6 / 9.1, 2560 x 4096 15.8 / 8.8, 11.7 / 8.6,
-	// 19456 x 2560 29.6 / 22.5, 27.8 / 19.0, 3072 x 2048 15.4 / 8.6, 8.4 / 7.4,
-	// but 2560 x 9728 23.3 / 13.2, 23.5 / 18.6 (X is read once per 16 rows
-	// there, four times the weights' bytes); BF16 3072 x 2048 12.7 / 8.4, 9.5 /
-	// 7.3, but 19456 x 2560 29.4 / 23.3, 33 / -. The lines are at numbers of
-	// columns, not of rows, so that a matrix gets the same bits alone and in a
-	// group.
+	// Up to 16 vectors run either kernel. Graph replays of one stream, us, 2 and 16
+	// vectors, gemv_kernel / gemv_batch_kernel (with its staging): BF16 2560 x
+	// 1024 10.9 / 6.7 and 12.2 / 6.8, 2560 x 2048 11.1 / 8.8 and 12.3 / 9.1, 6144 x
+	// 2048 12.3 / 12.2 and 14.3 / 12.4, 6144 x 2560 12.6 / 13.9 and 14.5 / 14.2 (and
+	// 14336 x 2048 18.4 / 20.4 and 21.3 / 20.7, the price of a line at columns);
+	// Q8_0 2560 x 2048 12.4 / 7.7 and 13.5 / 7.7, 6144 x 4096 18.8 / 17.1 and 22.1 /
+	// 17.2, 2560 x 6144 16.6 / 16.2 and 17.9 / 16.4, 2560 x 7168 17.5 / 18.2 and
+	// 19.1 / 18.5, 2560 x 9728, 16 vectors, 23.3 / 23.5 (X is read once per 16 rows
+	// there, four times the weights' bytes); Q4_S 6144 x 2048 13.1 / 10.5 and
+	// 14.5 / 10.5, 2560 x 6144 15.0 / 13.9 and 16.5 / 14.1, 2560 x 7168 15.5 / 16.2
+	// and 17.8 / 16.3. With three streams at once, which calls from one thread
+	// bound by their launches, two each, both take 7 to 8 us up to about 4096
+	// columns, and at 6144 two Q8_0 vectors 7.8 / 9.7 and sixteen 8.9 / 9.3. A
+	// narrow matrix takes gemv_kernel one launch and no scratch, 4.6 us of host
+	// time against 7.4: eager calls of one stream, 2 and 16 vectors, BF16 640 x 128
+	// 7.0 / 7.7 and 7.9 / 7.8, 4096 x 320 7.6 / 7.6 and 8.8 / 7.8; Q8_0 640 x 256
+	// 5.5 / 7.9 and 6.4 / 7.7, 4096 x 384 8.1 / 7.7 and 9.3 / 8.0; Q4_S 640 x 384
+	// 7.3 / 8.1 and 8.4 / 8.4, 2048 x 448 8.2 / 8.3 and 9.6 / 7.9 (replays of a graph,
+	// where the launch is cheap, 6.9 / 4.2 for BF16 640 x 128, 6.5 / 4.6 for Q8_0
+	// 640 x 384). The lines are at numbers of columns, not of rows, so that a
+	// matrix gets the same bits alone and in a group.
 	bool gemv_stages_x(int cols, int n_batch, int format)
 	{
 		if (gemv_vec_fits(cols, n_batch, format)) return false;
-		return n_batch > kGemvMaxBatch || cols <= (format == kGemvBf16 ? 2048 : 6144);
+		if (n_batch > kGemvMaxBatch) return true;
+		return format == kGemvBf16 ? cols > 256 && cols <= 2048 : cols > 384 && cols <= 6144;
 	}
 
 	// One launch takes all the vectors up to kGemvWideBatch, but where the kernel

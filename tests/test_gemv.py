@@ -570,6 +570,23 @@ def test_hip_gemv_many_vectors(orc, rows, cols, n):
                         hip_rt.free(d)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [256, 288, 384, 416, 2048, 2080, 6144, 6176])
+def test_hip_gemv_both_sides_of_the_staging_lines(orc, cols):
+    """2, 3 and 16 vectors at the columns where X begins and stops to be staged."""
+    import libllmcpu_amd as nh
+
+    rng = np.random.default_rng(cols)
+    wf = (rng.standard_normal((72, cols)) * 0.05).astype(np.float32)
+    x = (rng.standard_normal((16, cols)) * 2).astype(np.float32)
+    with nh.KVCache([16], [64]) as kv:
+        for fmt, wl in layouts(orc, wf).items():
+            for n in (2, 3, 16):
+                print(f"case gemv {fmt} 72 x {cols}, {n} vectors", flush=True)
+                got = kv.gemv(fmt, wl, x[:n], rows=72, cols=cols)
+                assert np.all(np.abs(got.astype(np.float64) - oracle_gemv(orc, fmt, wl, x[:n])) <= bound(fmt, wl, x[:n])), (fmt, n)
+
+
 # Few rows of many columns: 64 vectors at a time (a rest of 1, 6 and 32), and 16
 # at a time (a rest of 1 and 16).
 FEW_ROWS = [(40, 7168, 65), (129, 9760, 70), (72, 7200, 96), (24, 8800, 17), (33, 9728, 32)]

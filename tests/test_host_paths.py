@@ -136,6 +136,24 @@ def many_vectors_of_few_wide_rows(rt, nh):
                         assert group == want, (fmt, cols, n, rows, group, alone)
 
 
+@check
+def narrow_batches_are_one_launch(rt, nh):
+    """Up to 16 vectors of at most 256 (BF16) or 384 columns: one launch, no
+    scratch; beside the lines X is staged."""
+    for fmt in FORMATS:
+        last = 256 if fmt == "bf16" else 384
+        for cols in (32, 64, last, last + 32):
+            for n in (2, 3, 16):
+                with nh.KVCache([16], [64]) as kv:
+                    rt.clear()
+                    gemv(kv, fmt, n, 1000, cols)
+                    got = rt.launches()
+                    if cols <= last:
+                        assert route(got) == [("gemv_kernel", n, 1)] and not got[0]["scratch"], (fmt, cols, n)
+                    else:
+                        assert [r[0] for r in route(got)] == ["gemv_stage_x_kernel", "gemv_batch_kernel"], (fmt, cols, n)
+
+
 def attend(kv, n_tok, pos0=0, *, n_head=8, n_kv=8, head_dim=64):
     kv.attend_device(0, 1 << 20, 2 << 20, n_tok=n_tok, pos0=pos0, n_head=n_head, n_kv=n_kv, head_dim=head_dim, scale=0.1)
 
