@@ -1174,14 +1174,15 @@ namespace
 
 	// Vectors per launch of a gemv of n_batch, `most` by size; while the stream is
 	// captured into a graph and the scratch would have to grow (nothing can be
-	// allocated then), one, on the one-vector kernel.
-	static uint32_t gemv_chunk(const nnc_hip_kv* kv, int rows, int cols, uint32_t n_batch, int format, int most)
+	// allocated then), one, on the one-vector kernel. (A rest after the last
+	// whole launch can need more than they do: its K splits' partials.)
+	static uint32_t gemv_chunk(const nnc_hip_kv* kv, int rows, int cols, uint32_t n_batch, int format, uint32_t most)
 	{
 		if (n_batch == 1) return 1;
-		const int nb = static_cast<int>(std::min<uint32_t>(n_batch, most));
-		if (gemv_scratch_bytes(rows, cols, nb, format) > kv->gemv_part.bytes && nnchip::gemv_vec_fits(cols, 1, format) &&
-		    capturing(kv))
-			return 1;
+		size_t need = 0;
+		for (uint32_t nb : {std::min(n_batch, most), n_batch % most})
+			if (nb) need = std::max(need, gemv_scratch_bytes(rows, cols, static_cast<int>(nb), format));
+		if (need > kv->gemv_part.bytes && nnchip::gemv_vec_fits(cols, 1, format) && capturing(kv)) return 1;
 		return most;
 	}
 

@@ -154,6 +154,20 @@ def narrow_batches_are_one_launch(rt, nh):
                         assert [r[0] for r in route(got)] == ["gemv_stage_x_kernel", "gemv_batch_kernel"], (fmt, cols, n)
 
 
+@check
+def captured_batch_with_a_rest(rt, nh):
+    """A captured batch of whole launches and a rest finds the scratch of both
+    there, or runs a vector at a time: here the staged X of 1024 vectors was
+    reserved, and the rest of 16 needs more for its K splits."""
+    for warm in (1024, 1040):
+        with nh.KVCache([16], [64]) as kv:
+            gemv(kv, "bf16", warm, 1 << 16, 2560)
+            rt.clear()
+            rt.capture(lambda: gemv(kv, "bf16", 1040, 1 << 16, 2560))
+            got = {r[:2] for r in route(rt.launches())}
+            assert (got == {("gemv_vec_kernel", 1)}) == (warm == 1024), (warm, got)
+
+
 def attend(kv, n_tok, pos0=0, *, n_head=8, n_kv=8, head_dim=64):
     kv.attend_device(0, 1 << 20, 2 << 20, n_tok=n_tok, pos0=pos0, n_head=n_head, n_kv=n_kv, head_dim=head_dim, scale=0.1)
 
