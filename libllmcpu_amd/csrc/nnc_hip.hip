@@ -635,9 +635,21 @@ namespace
 	// windowed, us, one stream / three, tiled_kernel -> it: 300 tokens, 900 rows,
 	// 98 / 50 -> 123 / 55; 700 132 / 71 -> 149 / 70; 1024 162 / 85 -> 157 / 98;
 	// 1344, 4032 rows, 183 / 107 -> 169 / 91; 1700 196 / 125 -> 186 / 104; causal
-	// layers of 1000 tokens of 4 x 256, 4000 rows, 244 / 171 -> 197 / 123), as far
-	// as its scratch goes: kTiled3Scratch, and while the stream is captured
-	// (nothing can be allocated) what is there.
+	// layers of 1000 tokens of 4 x 256, 4000 rows, 244 / 171 -> 197 / 123). Its
+	// launches cost the same however few the keys, so rows x keys x head_dim
+	// (of whole blocks, all KV heads) must reach 270 million at head_dim 64 and
+	// 400 million above (us per layer, one stream / three: 32 heads over 8 x 64,
+	// 300 causal tokens, 92 million, 24 / 17 -> 29 / 20, 512 tokens, 269, 42 / 37
+	// -> 39 / 28; 8 over 8 x 128, 512 bidirectional tokens, 268, 29 / 23 -> 33 /
+	// 24, 1024 causal ones, 537, 62 / 57 -> 50 / 41). The operands take three
+	// times the keys' bytes out of kTiled3Scratch, and where the partials of as
+	// many splits as fill the chip no longer fit beside them, the splits that do
+	// must still give work to half the CUs at head_dim 256 (eight wavefronts
+	// each) and three quarters below (8 over 8 x 128, 512 tokens over 2000 keys,
+	// one split, 32 work-groups: 74 / 62 -> 209 / 151; 8 over 8 x 256, 1024 causal
+	// tokens, 64: 95 / 83 -> 150 / 103; but 8 over 2 x 256, 2048 tokens, 128: 0.87
+	// of the time, 32 over 8 x 128, 768 tokens, 192: 0.77). While the stream is
+	// captured (nothing can be allocated) the scratch is what is there.
 	void plan_tiled(const nnc_hip_kv* kv, int32_t n_tok, int32_t pos0, int32_t n_seq, int32_t window, bool causal,
 	                int32_t n_kv, int32_t head_dim, int group, const part_source& src, std::vector<decode_plan>& plan)
 	{
@@ -645,8 +657,10 @@ namespace
 		{
 			const int32_t nt = std::min(kTiledChunk, n_tok - t0);
 			const long long n_rows = static_cast<long long>(nt) * group;
+			long long row_keys = 0, wanted = 0; // of the last make(): rows x keys of a KV head's blocks; splits to fill the part
 			auto make = [&](int block, int align, int per_cu, long long max_splits)
 			{
+				row_keys = 0;
 				const long long n_blk = (n_rows + block - 1) / block;
 				std::vector<int> spans(static_cast<size_t>(n_blk));
 				int max_span = 1;
@@ -658,10 +672,11 @@ namespace
 					nnchip::attn_span(causal ? 1 : 0, window, pos0 + t0 + static_cast<int32_t>(r1 / group), n_seq, unused, hi);
 					lo = lo / align * align;
 					spans[static_cast<size_t>(blk)] = std::max(0, hi - lo + 1);
+					row_keys += static_cast<long long>(block) * spans[static_cast<size_t>(blk)];
 					max_span = std::max(max_span, hi - lo + 1);
 				}
-				const long long want =
-					std::min(max_splits, std::max<long long>(1, 1LL * kv->n_cu * per_cu / (n_blk * n_kv)));
+				wanted = std::max<long long>(1, 1LL * kv->n_cu * per_cu / (n_blk * n_kv));
+				const long long want = std::min(max_splits, wanted);
 				const int step = std::max(align, 16);
 				long long sk = (max_span + want - 1) / want;
 				sk = std::max<long long>(64, (sk + step - 1) / step * step);
@@ -687,7 +702,11 @@ namespace
 					d.k_hi = k_hi;
 					const size_t need = split + tiled_part_bytes(d, group * n_kv, n_kv, head_dim);
 					const bool there = src.ptr ? need <= src.bytes : need <= kv->part.bytes || !capturing(kv);
-					if (need <= kTiled3Scratch && there)
+					const long long least = head_dim == 64 ? 270000000 : 400000000;
+					const long long n_blk = (n_rows + nnchip::kTiled3Block - 1) / nnchip::kTiled3Block;
+					const bool filled =
+						room >= wanted || n_blk * n_kv * room >= (head_dim == 256 ? kv->n_cu / 2 : kv->n_cu * 3 / 4);
+					if (need <= kTiled3Scratch && row_keys * n_kv * head_dim >= least && filled && there)
 					{
 						plan.push_back(d);
 						continue;

@@ -113,10 +113,11 @@ def test_tiled_noalloc_matches_attend_device(orc):
     assert errors(a, want)[0] <= 1e-3
 
 
-# Both sides of the rule for the three-part bf16 products (512 rows per KV head
-# and 4000 in all; 128-row blocks, 32-key groups): the smallest batch that takes
-# them and one token less, ragged last blocks, one split and many, windows on
-# both sides, rings that have wrapped, spans that start mid-group.
+# Both sides of the rule for the three-part bf16 products (512 rows per KV head,
+# 4000 in all and enough keys; 128-row blocks, 32-key groups): the smallest
+# batch that takes them and one token less, ragged last blocks, one split and
+# many, windows on both sides, rings that have wrapped, spans that start
+# mid-group.
 T3_CASES = (
     # n_head, n_kv, head_dim, causal, window, n_seq, n_tok, ring
     (4, 1, 256, True, 0, 1011, 1000, False),
@@ -128,6 +129,13 @@ T3_CASES = (
     (8, 2, 64, True, 0, 555, 501, False),
     (32, 8, 64, False, 200, 150, 150, False),
     (4, 4, 256, True, 700, 2600, 1003, True),
+    # (the cases above of little work, or whose operands leave no room for
+    # splits, run the fp32 products; these the three-part ones)
+    (4, 1, 256, True, 700, 2600, 1003, True),
+    (16, 8, 128, True, 300, 1500, 900, True),
+    (8, 2, 64, True, 600, 2600, 1003, True),
+    (8, 2, 64, True, 0, 1055, 1001, False),
+    (32, 8, 64, False, 400, 600, 600, False),
 )
 
 

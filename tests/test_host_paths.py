@@ -168,8 +168,27 @@ def captured_batch_with_a_rest(rt, nh):
             assert (got == {("gemv_vec_kernel", 1)}) == (warm == 1024), (warm, got)
 
 
-def attend(kv, n_tok, pos0=0, *, n_head=8, n_kv=8, head_dim=64):
-    kv.attend_device(0, 1 << 20, 2 << 20, n_tok=n_tok, pos0=pos0, n_head=n_head, n_kv=n_kv, head_dim=head_dim, scale=0.1)
+def attend(kv, n_tok, pos0=0, *, n_head=8, n_kv=8, head_dim=64, causal=True, window=0):
+    kv.attend_device(0, 1 << 20, 2 << 20, n_tok=n_tok, pos0=pos0, n_head=n_head, n_kv=n_kv, head_dim=head_dim, scale=0.1,
+                     causal=causal, window=window)
+
+
+@check
+def long_f32_batches_take_the_kernel_that_is_faster(rt, nh):
+    """The three-part products from enough work on, and only where their operands
+    leave room for the splits that fill the chip."""
+    three = [(32, 8, 64, 0, 512, True, 0), (8, 8, 128, 0, 1024, True, 0), (3, 1, 256, 0, 2048, False, 512),
+             (4, 1, 256, 0, 1000, True, 0), (32, 8, 128, 0, 768, True, 0), (8, 2, 256, 0, 2048, False, 0)]
+    fp32 = [(32, 8, 64, 0, 300, True, 0), (16, 8, 128, 0, 300, True, 0), (8, 8, 128, 0, 512, False, 0),
+            (8, 8, 128, 2000, 512, True, 0), (16, 8, 128, 2000, 512, True, 0), (8, 8, 256, 0, 1024, True, 0),
+            (8, 2, 256, 2000, 1024, True, 0), (4, 1, 256, 0, 999, True, 0)]
+    for cases, kernel in ((three, "tiled3_kernel"), (fp32, "12tiled_kernel")):
+        for n_head, n_kv, hd, pos0, n, causal, window in cases:
+            with nh.KVCache([4096], [n_kv * hd], bf16=False) as kv:
+                rt.clear()
+                attend(kv, n, pos0, n_head=n_head, n_kv=n_kv, head_dim=hd, causal=causal, window=window)
+                names = [l["name"] for l in rt.launches()]
+                assert any(kernel in m for m in names), (n_head, n_kv, hd, pos0, n, names)
 
 
 @check
