@@ -644,12 +644,13 @@ namespace
 	// 24, 1024 causal ones, 537, 62 / 57 -> 50 / 41). The operands take three
 	// times the keys' bytes out of kTiled3Scratch, and where the partials of as
 	// many splits as fill the chip no longer fit beside them, the splits that do
-	// must still give work to half the CUs at head_dim 256 (eight wavefronts
+	// must still give work to a third of the CUs at head_dim 256 (eight wavefronts
 	// each) and three quarters below (8 over 8 x 128, 512 tokens over 2000 keys,
 	// one split, 32 work-groups: 74 / 62 -> 209 / 151; 8 over 8 x 256, 1024 causal
-	// tokens, 64: 95 / 83 -> 150 / 103; but 8 over 2 x 256, 2048 tokens, 128: 0.87
-	// of the time, 32 over 8 x 128, 768 tokens, 192: 0.77). While the stream is
-	// captured (nothing can be allocated) the scratch is what is there.
+	// tokens, 64: 95 / 83 -> 150 / 103; but 8 over 2 x 256, 1500 tokens, 94: causal
+	// 195 / 147 -> 209 / 140, bidirectional 239 / 191 -> 211 / 142; 32 over 8 x 128,
+	// 768 tokens, 192: 0.77 of the time). While the stream is captured (nothing
+	// can be allocated) the scratch is what is there.
 	void plan_tiled(const nnc_hip_kv* kv, int32_t n_tok, int32_t pos0, int32_t n_seq, int32_t window, bool causal,
 	                int32_t n_kv, int32_t head_dim, int group, const part_source& src, std::vector<decode_plan>& plan)
 	{
@@ -694,9 +695,9 @@ namespace
 				if (split <= kTiled3Scratch)
 				{
 					const size_t row_bytes = static_cast<size_t>(n_rows) * n_kv * (head_dim + 4) * sizeof(float); // per split
-					const long long room = static_cast<long long>((kTiled3Scratch - split) / row_bytes);
-					decode_plan d = make(nnchip::kTiled3Block, nnchip::kTiled3Keys, head_dim == 256 ? 1 : 2,
-					                     std::max<long long>(room, 1));
+					const long long room = // (one split needs none)
+						std::max<long long>(1, static_cast<long long>((kTiled3Scratch - split) / row_bytes));
+					decode_plan d = make(nnchip::kTiled3Block, nnchip::kTiled3Keys, head_dim == 256 ? 1 : 2, room);
 					d.split_bytes = split;
 					d.k_lo = k_lo;
 					d.k_hi = k_hi;
@@ -705,7 +706,7 @@ namespace
 					const long long least = head_dim == 64 ? 270000000 : 400000000;
 					const long long n_blk = (n_rows + nnchip::kTiled3Block - 1) / nnchip::kTiled3Block;
 					const bool filled =
-						room >= wanted || n_blk * n_kv * room >= (head_dim == 256 ? kv->n_cu / 2 : kv->n_cu * 3 / 4);
+						room >= wanted || n_blk * n_kv * room >= (head_dim == 256 ? kv->n_cu / 3 : kv->n_cu * 3 / 4);
 					if (need <= kTiled3Scratch && row_keys * n_kv * head_dim >= least && filled && there)
 					{
 						plan.push_back(d);
