@@ -179,7 +179,8 @@ def long_f32_batches_take_the_kernel_that_is_faster(rt, nh):
     leave room for the splits that fill the chip."""
     three = [(32, 8, 64, 0, 512, True, 0), (8, 8, 128, 0, 1024, True, 0), (3, 1, 256, 0, 2048, False, 512),
              (4, 1, 256, 0, 1000, True, 0), (32, 8, 128, 0, 768, True, 0), (8, 2, 256, 0, 2048, False, 0),
-             (16, 8, 128, 0, 2048, True, 0), (32, 8, 64, 2000, 2048, True, 0)]
+             (16, 8, 128, 0, 2048, True, 0), (32, 8, 64, 2000, 2048, True, 0),
+             (8, 2, 256, 0, 1500, False, 0)]
     fp32 = [(32, 8, 64, 0, 300, True, 0), (16, 8, 128, 0, 300, True, 0), (8, 8, 128, 0, 512, False, 0),
             (8, 8, 128, 2000, 512, True, 0), (16, 8, 128, 2000, 512, True, 0), (8, 8, 256, 0, 1024, True, 0),
             (8, 2, 256, 2000, 1024, True, 0), (4, 1, 256, 0, 999, True, 0)]
