@@ -380,32 +380,49 @@ namespace nnchip
 		// the operands' kernel and the merge around them.
 		constexpr int kT3Block = kTiled3Block, kT3Keys = kTiled3Keys;
 
-		// x as bf16 parts, x = out[0] + out[1] + out[2] to 24 bits. ANY (K, V and
-		// Q; the weights are at most 2^8): a part holds at most the largest finite
-		// bf16, so a finite x near the fp32 limit stays finite, an infinite one is
-		// (largest, largest, inf), whose products with an operand are infinite of
-		// the right sign or finite, and NaN stays in the last part.
-		template <bool ANY>
+		// x as bf16 parts, x = out[0] + out[1] + out[2] to 24 bits (fewer below
+		// 2^-109, where the last is subnormal). Parts are at most the largest
+		// finite bf16: the first for K and V, which are finite wherever the parts
+		// are used; for Q the second too, so an infinite x is (largest, largest,
+		// x), whose products with elements below 2^8 are infinite of the right
+		// sign or finite. NaN stays in the last part. (The weights: at most 2^8.)
+		enum t3_operand { kT3KV, kT3Q, kT3P };
+		template <t3_operand OF>
 		__device__ __forceinline__ void split3(const float (&x)[8], u32x4 (&out)[3])
 		{
 			const float big = __uint_as_float(0x7f7f0000u);
-			auto lim = [&](float v) __attribute__((always_inline)) { return ANY ? fminf(fmaxf(v, -big), big) : v; };
+			auto lim = [&](bool on, float v) __attribute__((always_inline)) { return on ? __builtin_amdgcn_fmed3f(v, -big, big) : v; };
 #pragma unroll
 			for (int j = 0; j < 4; ++j)
 			{
 				const float a = x[2 * j], b = x[2 * j + 1];
-				const uint32_t h = cvt_pk_bf16(lim(a), lim(b));
+				const uint32_t h = cvt_pk_bf16(lim(OF != kT3P, a), lim(OF != kT3P, b));
 				const float a1 = a - bf16_lo(h), b1 = b - bf16_hi(h);
-				const uint32_t m = cvt_pk_bf16(lim(a1), lim(b1));
+				const uint32_t m = cvt_pk_bf16(lim(OF == kT3Q, a1), lim(OF == kT3Q, b1));
 				out[0][j] = h;
 				out[1][j] = m;
 				out[2][j] = cvt_pk_bf16(a1 - bf16_lo(m), b1 - bf16_hi(m));
 			}
 		}
 
+		// z stays 0 while every x is finite, and is NaN once one is not.
+		__device__ __forceinline__ void add_zeros(const float (&x)[8], float& z)
+		{
+#pragma unroll
+			for (int j = 0; j < 8; ++j) z = fmaf(x[j], 0.0f, z);
+		}
+
 		// Bytes of a group's K (or V) of one head.
 		template <int HD>
 		constexpr uint32_t kT3Bytes = HD * kT3Keys * 6;
+
+		// After the operands: per (head, group) whether K or V holds an infinite
+		// or NaN element, one word for each wavefront of tiled3_split_kernel.
+		template <int HD>
+		__device__ __forceinline__ uint4* t3_flags(char* split, int n_kv, int n_g, int kvh)
+		{
+			return reinterpret_cast<uint4*>(split + static_cast<size_t>(n_kv) * n_g * 2 * kT3Bytes<HD>) + static_cast<size_t>(kvh) * n_g;
+		}
 
 		// Group g0 + blockIdx.x of head blockIdx.y; keys outside k_lo .. k_hi as
 		// zeros.
@@ -418,6 +435,7 @@ namespace nnchip
 			auto row = [&](int k) { return static_cast<size_t>(k % p.rows) * p.kv_dim + head_off; };
 			const float* K = static_cast<const float*>(p.K);
 			const float* V = static_cast<const float*>(p.V);
+			float z = 0.0f;
 			for (int i = threadIdx.x; i < HD * 4; i += 256) // (8 elements each)
 			{
 				const int lane = i & 63, f = i >> 6, r = lane & 15, g = lane >> 4;
@@ -434,7 +452,8 @@ namespace nnchip
 					}
 					x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
 					x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
-					split3<true>(x, o);
+					add_zeros(x, z);
+					split3<kT3KV>(x, o);
 #pragma unroll
 					for (int c = 0; c < 3; ++c) *reinterpret_cast<u32x4*>(dst + (f * 3 + c) * 1024 + 16 * lane) = o[c];
 				}
@@ -445,12 +464,16 @@ namespace nnchip
 						const int k = key0 + 16 * (j >> 2) + 4 * g + (j & 3);
 						x[j] = k >= k_lo && k <= k_hi ? V[row(k) + 16 * f + r] : 0.0f;
 					}
-					split3<true>(x, o);
+					add_zeros(x, z);
+					split3<kT3KV>(x, o);
 #pragma unroll
 					for (int c = 0; c < 3; ++c)
 						*reinterpret_cast<u32x4*>(dst + kT3Bytes<HD> + (f * 3 + c) * 1024 + 16 * lane) = o[c];
 				}
 			}
+			const bool any = __builtin_amdgcn_ballot_w64(z != 0.0f) != 0;
+			if ((threadIdx.x & 63) == 0)
+				reinterpret_cast<uint32_t*>(t3_flags<HD>(split, p.n_kv, gridDim.x, kvh) + blockIdx.x)[threadIdx.x >> 6] = any;
 		}
 
 		__device__ __forceinline__ void t3_dma(__amdgpu_buffer_rsrc_t r, unsigned char* dst, uint32_t off, uint32_t s_off)
@@ -494,6 +517,67 @@ namespace nnchip
 					for (int y = 0; y < NA; ++y) c[y][x] = mfma16x16x32(as_bf16x8(a[x][A[u]]), as_bf16x8(b[y][B[u]]), c[y][x]);
 		}
 
+		// Rows row .. end - 1 (one wavefront's) over keys w_lo .. w_hi of their own
+		// spans, in fp32, a row at a time: the work-groups whose keys hold an
+		// infinite or NaN element of K or V. In the matrix products a key that
+		// weighs 0 in a row makes it NaN all the same, and the parts of an
+		// infinite operand have no right products with the other's lower parts.
+		template <int HD>
+		__device__ void t3_rows_fp32(const decode_params& p, int G, int kvh, int z, int row, int end, int w_lo, int w_hi)
+		{
+			constexpr int E = HD / 64;
+			const int e0 = E * (threadIdx.x & 63);
+			const float* K = static_cast<const float*>(p.K) + static_cast<size_t>(kvh) * HD + e0;
+			const float* V = static_cast<const float*>(p.V) + static_cast<size_t>(kvh) * HD + e0;
+			for (; row < end; ++row)
+			{
+				const int t = row / G, h = row % G;
+				const size_t qo = (static_cast<size_t>(t) * p.n_head + static_cast<size_t>(kvh) * G + h) * HD + e0;
+				int first, last;
+				attn_span(p.causal, p.window, p.pos0 + t, p.n_seq, first, last);
+				float q[E], o[E], m = -INFINITY, l = 0.0f;
+#pragma unroll
+				for (int e = 0; e < E; ++e)
+				{
+					q[e] = p.q[qo + e] * p.qscale;
+					o[e] = 0.0f;
+				}
+				for (int k = max(first, w_lo); k <= min(last, w_hi); ++k)
+				{
+					const size_t at = static_cast<size_t>(k % p.rows) * p.kv_dim;
+					float s = 0.0f;
+#pragma unroll
+					for (int e = 0; e < E; ++e) s = fmaf(q[e], K[at + e], s);
+					s = wave_sum_dpp(s);
+					if (s > m + kTileLazy)
+					{
+						const float alpha = m == -INFINITY ? 1.0f : fast_exp2(m - s);
+						m = s;
+						l *= alpha;
+#pragma unroll
+						for (int e = 0; e < E; ++e) o[e] *= alpha;
+					}
+					const float w = fast_exp2(s - (m == -INFINITY ? 0.0f : m));
+					l += w;
+#pragma unroll
+					for (int e = 0; e < E; ++e) o[e] = fmaf(w, V[at + e], o[e]);
+				}
+				if (p.n_split > 1)
+				{
+					float* gp = tiled_partial(p, G, HD, t, kvh, z, h);
+#pragma unroll
+					for (int e = 0; e < E; ++e) gp[e0 + e] = o[e];
+					if (e0 == 0) *reinterpret_cast<float2*>(gp + HD) = make_float2(m, l);
+				}
+				else
+				{
+					const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+#pragma unroll
+					for (int e = 0; e < E; ++e) p.out[qo + e] = gated(o[e] * inv, p.gate, qo + e);
+				}
+			}
+		}
+
 		// Row tiles per wavefront: two at head_dim 64 and 128 (a fragment read
 		// from LDS serves two products; four wavefronts, two work-groups per
 		// CU), one at 256, where two tiles' Q and O left one wavefront per SIMD and
@@ -535,6 +619,16 @@ namespace nnchip
 			load(0, 0, s_k);
 			load(0, 1, s_v);
 
+			uint32_t bad = 0; // of a lane, not 0: an infinite or NaN element in these keys' K or V
+			{
+				const uint4* flags = t3_flags<HD>(const_cast<char*>(split), p.n_kv, n_g, kvh) + (w_lo / kT3Keys - g0);
+				for (int i = lane; i < n_steps; i += 64)
+				{
+					const uint4 f = flags[i];
+					bad |= f.x | f.y | f.z | f.w;
+				}
+			}
+
 			// This lane's row of each of the wavefront's tiles.
 			int r_lo[NA], r_hi[NA];
 			size_t qo[NA];
@@ -557,7 +651,7 @@ namespace nnchip
 					const float4 v = *reinterpret_cast<const float4*>(p.q + qo[a] + 32 * kk + 8 * c + 4);
 					const float x[8] = {u.x * p.qscale, u.y * p.qscale, u.z * p.qscale, u.w * p.qscale,
 					                    v.x * p.qscale, v.y * p.qscale, v.z * p.qscale, v.w * p.qscale};
-					split3<true>(x, q[kk][a]);
+					split3<kT3Q>(x, q[kk][a]);
 				}
 			}
 
@@ -574,6 +668,12 @@ namespace nnchip
 			// (Q's loads came after the first DMAs: none of this is counted on)
 			__builtin_amdgcn_sched_barrier(0);
 			__builtin_amdgcn_s_waitcnt(0x0F70);
+			if (__builtin_amdgcn_ballot_w64(bad != 0)) // (the same in every wavefront)
+			{
+				const int row = blockIdx.x * kT3Block + 16 * NA * wave;
+				t3_rows_fp32<HD>(p, G, kvh, z, row, min(row + 16 * NA, n_rows), w_lo, w_hi);
+				return;
+			}
 
 			for (int st = 0; st < n_steps; ++st)
 			{
@@ -644,7 +744,7 @@ namespace nnchip
 						ls += w[j];
 					}
 					l_run[a] += row4_sum(ls);
-					split3<false>(w, pw[a]);
+					split3<kT3P>(w, pw[a]);
 				}
 
 				t3_wait_barrier<ND>(); // V has landed; the next K may be in flight

@@ -110,9 +110,10 @@ namespace nnchip
 
 	// The same batches of F32 caches at head_dim 64, 128 and 256 with the
 	// products as sums of six bf16 ones (24 bits): the span's K and V (keys
-	// k_lo .. k_hi) are first written to `split` as matrix operands,
-	// tiled3_bytes of them. Row blocks of 128, splits of a multiple of 32 keys
-	// relative to the block's first key rounded down to 32.
+	// k_lo .. k_hi) are first written to `split` as matrix operands, with a flag
+	// per 32 keys and KV head for infinite and NaN elements, tiled3_bytes in
+	// all. Row blocks of 128, splits of a multiple of 32 keys relative to the
+	// block's first key rounded down to 32.
 	constexpr int kTiled3Block = 128, kTiled3Keys = 32;
 	__host__ __device__ inline bool tiled3_shape(int head_dim)
 	{
@@ -120,7 +121,8 @@ namespace nnchip
 	}
 	inline size_t tiled3_bytes(int k_lo, int k_hi, int n_kv, int head_dim)
 	{
-		return static_cast<size_t>(k_hi / kTiled3Keys - k_lo / kTiled3Keys + 1) * n_kv * head_dim * kTiled3Keys * 12;
+		return static_cast<size_t>(k_hi / kTiled3Keys - k_lo / kTiled3Keys + 1) * n_kv *
+		       (static_cast<size_t>(head_dim) * kTiled3Keys * 12 + 16);
 	}
 	bool launch_tiled3(const decode_params& p, int n_tok, int head_dim, int group, void* split, int k_lo, int k_hi,
 	                   hipStream_t stream);

@@ -236,3 +236,61 @@ def test_f32_three_part_special_values():
     ok = np.isfinite(want)
     g, w = got[ok].astype(np.float64), want[ok].astype(np.float64)
     assert (np.abs(g - w) <= 2e-5 * (1 + np.abs(w))).all()
+
+
+@pytest.mark.parametrize("c", ((4, 1, 256, True, 0), (4, 1, 256, True, 420), (16, 8, 128, True, 0), (16, 8, 128, False, 400),
+                               (8, 8, 64, True, 0), (16, 8, 64, False, 401)), ids=lambda c: "-".join(map(str, c)))
+def test_f32_three_part_non_finite_v_stays_with_its_rows(c):
+    """An infinite or NaN V row changes no token that does not attend it (to 2e-5:
+    the rows of a work-group that has such a key run in fp32), whichever block,
+    key group or split the key shares with it; those that attend it are not finite."""
+    n_head, n_kv, hd, causal, window = c
+    n = 1100
+    cfg = synth.AttnConfig(65, "t3 reach", n_head, n_kv, hd, 1, kv_bf16=False, window=window, swa_period=2)
+    K, V = synth.cache_buffer(cfg, 0, n, n)
+    q = synth.qk_rows(cfg, 0, 0, np.arange(n), n_head)
+    kw = dict(pos0=0, n_seq=n, window=window, causal=causal, n_head=n_head, n_kv=n_kv, head_dim=hd, scale=cfg.attn_scale)
+    span = [nh.attn_span(causal, window, t, n) for t in range(n)]
+    with nh.KVCache([n], [cfg.kv_dim], bf16=False) as kv:
+        say(f"case three-part reach of non-finite V {c}")
+        kv.append(0, 0, K, V)
+        want = kv.attend(0, q, **kw)
+        for k, x in ((333, np.inf), (511, np.nan), (640, -np.inf), (1003, np.nan)):
+            kv.append(0, k, K[k:k + 1], np.full_like(V[k:k + 1], x))
+            got = kv.attend(0, q, **kw)
+            kv.append(0, k, K[k:k + 1], V[k:k + 1])
+            dirty = np.array([lo <= k <= hi for lo, hi in span])
+            same = (np.abs(got - want) <= 2e-5 * (1 + np.abs(want))).all(1)
+            say(f"  key {k}: attended by {dirty.sum()} tokens; others changed {np.flatnonzero(~dirty & ~same)[:40]}")
+            assert (~dirty).sum() > 50 and same[~dirty].all()
+            assert not np.isfinite(got[dirty]).any()
+
+
+def test_f32_three_part_infinite_scores():
+    """Infinite K against large Q elements, and infinite Q against large K ones, of
+    either sign in their second bf16 part: scores of -inf weigh 0 and rows whose
+    every score is -inf are 0, as in shorter batches, which run fp32 products."""
+    n_head, n_kv, hd, n = 4, 1, 256, 1024
+    cfg = synth.AttnConfig(66, "t3 infinite scores", n_head, n_kv, hd, 1, kv_bf16=False)
+    K, V = synth.cache_buffer(cfg, 0, n, n)
+    q = synth.qk_rows(cfg, 0, 0, np.arange(n), n_head)
+    rng = np.random.default_rng(4)
+    large = (rng.uniform(4e3, 9e4, (n, n_head))).astype(np.float32)
+    kw = dict(n_seq=n, causal=False, n_head=n_head, n_kv=n_kv, head_dim=hd, scale=cfg.attn_scale)
+    for what in ("K", "Q"):
+        k1, q1 = K.copy(), q.copy()
+        if what == "K":
+            k1[:, 9], k1[55, 9] = 0, -np.inf
+            q1.reshape(n, n_head, hd)[:, :, 9] = large
+        else:
+            k1[:, 9] = -large[:, 0] / 512  # (below 2^8)
+            q1.reshape(n, n_head, hd)[:, :, 9] = 0
+            q1.reshape(n, n_head, hd)[::7, :, 9] = np.inf
+        say(f"case three-part infinite {what}")
+        with nh.KVCache([n], [cfg.kv_dim], bf16=False) as kv:
+            kv.append(0, 0, k1, V)
+            got = kv.attend(0, q1, pos0=0, **kw)
+            want = np.concatenate([kv.attend(0, q1[i:i + 256], pos0=i, **kw) for i in range(0, n, 256)])
+        assert np.isfinite(want).all()
+        assert (np.abs(got - want) <= 2e-5 * (1 + np.abs(want))).all(), what
+        assert what == "K" or (want[::7] == 0).all()
