@@ -478,12 +478,17 @@ namespace nnchip
 				if (lane < 16)
 				{
 					uint16_t* o = x_sums(p, blk >> 5, tile) + (lane + 16 * ((blk & 31) >> 3)) * 8 + (blk & 7);
-					const uint32_t h = f32_to_bf16_bits(s);
-					const float r = s - bf16_bits_to_f32(h);
+					// (the first part at most the largest finite bf16; an infinite
+					// sum or NaN is every part)
+					const float big = bf16_bits_to_f32(0x7f7f);
+					const bool finite = fabsf(s) < INFINITY;
+					if (s != s) s = __uint_as_float(0x7fc00000u); // (whose rounding stays NaN)
+					const uint32_t h = f32_to_bf16_bits(finite ? fminf(fmaxf(s, -big), big) : s);
+					const float r = finite ? s - bf16_bits_to_f32(h) : s;
 					const uint32_t m = f32_to_bf16_bits(r);
 					o[0] = static_cast<uint16_t>(h);
 					o[512] = static_cast<uint16_t>(m);
-					o[1024] = static_cast<uint16_t>(f32_to_bf16_bits(r - bf16_bits_to_f32(m)));
+					o[1024] = static_cast<uint16_t>(f32_to_bf16_bits(finite ? r - bf16_bits_to_f32(m) : s));
 				}
 			}
 		}

@@ -587,6 +587,34 @@ def test_hip_gemv_both_sides_of_the_staging_lines(orc, cols):
                 assert np.all(np.abs(got.astype(np.float64) - oracle_gemv(orc, fmt, wl, x[:n])) <= bound(fmt, wl, x[:n])), (fmt, n)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 16, 40, 70])
+def test_hip_gemv_q4_s_block_sums_at_the_limit(orc, n):
+    """The caller's block sums, as large as fp32 holds and infinite: every kernel
+    gives bias x sum as fp32 products do, by class, and the finite ones within
+    the bound."""
+    import libllmcpu_amd as nh
+
+    rng = np.random.default_rng(n)
+    rows, cols = 48, 1056
+    qs, sc, bi = layouts(orc, (rng.standard_normal((rows, cols)) * 0.05).astype(np.float32))["q4_s"]
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    with nh.KVCache([16], [64]) as kv:
+        for value in (3.4e38, -3.4e38, np.inf, -np.inf, np.nan):
+            xs = orc.block_sums(x).copy()
+            xs[n // 2, 17] = value
+            print(f"case gemv q4_s block sum {value}, {n} vectors", flush=True)
+            got = kv.gemv("q4_s", (qs, sc, bi), x, rows=rows, cols=cols, xsum=xs)
+            plain = kv.gemv("q4_s", (qs, sc, bi), x, rows=rows, cols=cols)
+            others = np.arange(n) != n // 2
+            assert np.array_equal(got[others], plain[others])
+            want = nh.bf16_to_f32(bi[:, 17]).astype(np.float64) * value
+            if np.isfinite(value):
+                assert np.all(np.abs(got[n // 2] - want) <= 1e-5 * np.abs(want) + 1e3)
+            else:
+                assert np.array_equal(got[n // 2].astype(np.float64), want, equal_nan=True)
+
+
 # Few rows of many columns: 64 vectors at a time (a rest of 1, 6 and 32), and 16
 # at a time (a rest of 1 and 16).
 FEW_ROWS = [(40, 7168, 65), (129, 9760, 70), (72, 7200, 96), (24, 8800, 17), (33, 9728, 32)]
