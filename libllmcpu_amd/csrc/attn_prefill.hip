@@ -229,12 +229,17 @@ namespace nnchip
 		}
 
 		// OCC wavefronts per SIMD. At head_dim 64 a work-group takes 80 KiB of LDS,
-		// so two share a CU when their registers allow (OCC = 4, 128 each): a
-		// 1024-token chunk of Llama-3.2-1B 19.7 -> 14.0 us per layer, 512 tokens
-		// over 4000 keys 33.0 -> 27.1 with three streams at once. In a launch
-		// that leaves most CUs with one work-group or none the narrower register
-		// budget only costs (64 tokens, 32 work-groups: 4 % per call), so OCC = 2
-		// runs those.
+		// so two share a CU when their registers allow (OCC = 4, 128 each). Above
+		// 256 work-groups the second one hides the first's loads (us per layer of
+		// 32 heads over 8, OCC = 2 / 4, one stream and three at once: 514 tokens,
+		// 264 work-groups, 22.8 / 18.4 and 12.2 / 9.3; 1024 tokens 31.3 / 23.4 and
+		// 25.8 / 19.7). Up to 256 a stream by itself gives each CU one, and the
+		// narrower register budget only costs: 3 % (317 tokens, 160 work-groups,
+		// 13.7 / 14.1; 384 14.0 / 14.4; 512, 256 of them, 15.5 / 15.9; in graph
+		// replays, without the gaps between launches, up to 9 %). But other
+		// streams' work-groups then find room: 7.2 / 6.4, 8.5 / 7.1 and 11.3 / 9.0
+		// with three, 11 to 20 % less. So the line is where that begins, 128
+		// work-groups (256 tokens: 12.7 / 12.9 and 6.2 / 6.2).
 		template <int HD, int G, int RG, int OCC>
 		__global__ __launch_bounds__(64 * kKG * RG) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void prefill_kernel(
 			const prefill_params p)
