@@ -476,12 +476,6 @@ namespace nnchip
 				reinterpret_cast<uint32_t*>(t3_flags<HD>(split, p.n_kv, gridDim.x, kvh) + blockIdx.x)[threadIdx.x >> 6] = any;
 		}
 
-		__device__ __forceinline__ void t3_dma(__amdgpu_buffer_rsrc_t r, unsigned char* dst, uint32_t off, uint32_t s_off)
-		{
-			typedef __attribute__((address_space(3))) void* lds_ptr;
-			__builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)dst, 16, off, s_off, 0, 0);
-		}
-
 		// At most N of this wavefront's loads in flight (s_waitcnt vmcnt(N), the
 		// other counters not waited on), then everyone's.
 		template <int N>
@@ -614,7 +608,7 @@ namespace nnchip
 				const uint32_t o = st < n_steps ? (static_cast<uint32_t>(w_lo / kT3Keys - g0 + st) * 2 + v) * kT3Bytes<HD> : 0u;
 				const uint32_t lo = st < n_steps ? 16u * lane + 1024u * wave : 0x80000000u;
 #pragma unroll
-				for (int u = 0; u < ND; ++u) t3_dma(rs, dst + 1024 * (NWV * u + wave), lo, o + 1024 * NWV * u);
+				for (int u = 0; u < ND; ++u) dma_lds16(rs, dst + 1024 * (NWV * u + wave), lo, o + 1024 * NWV * u);
 			};
 			load(0, 0, s_k);
 			load(0, 1, s_v);

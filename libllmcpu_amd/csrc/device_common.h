@@ -86,6 +86,14 @@ namespace nnchip
 		return add_with_other_half(x);
 	}
 
+	// 16 bytes per lane from byte off + s_off of the buffer to LDS, 1 KB from
+	// dst on in lane order.
+	__device__ __forceinline__ void dma_lds16(__amdgpu_buffer_rsrc_t r, unsigned char* dst, uint32_t off, uint32_t s_off)
+	{
+		typedef __attribute__((address_space(3))) void* lds_ptr;
+		__builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)dst, 16, off, s_off, 0, 0);
+	}
+
 	// 16 bytes with the non-temporal hint (global_load_dwordx4 ... nt): for
 	// K/V rows that one call reads once. Measured on a 134 MB per-head-slice
 	// stream: 22.4 us with the hint, 25.2 us without.

@@ -493,14 +493,6 @@ namespace nnchip
 			}
 		}
 
-		// 16 bytes per lane from byte off + s_off of the buffer to LDS, 1 KB from
-		// dst on in lane order.
-		__device__ __forceinline__ void dma_lds16(__amdgpu_buffer_rsrc_t r, unsigned char* dst, uint32_t off, uint32_t s_off)
-		{
-			typedef __attribute__((address_space(3))) void* lds_ptr;
-			__builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)dst, 16, off, s_off, 0, 0);
-		}
-
 		// 16 rows of each of RT tiles (rows past the last one repeat it; they are
 		// not stored), read through one buffer descriptor per tile. A piece goes
 		// to LDS by LDS-DMA with four lanes on each row's 64 bytes (row l / 4),
@@ -1009,8 +1001,9 @@ namespace nnchip
 		// Whether a row pair's last chunk is one item for both rows: when it is at
 		// most half full, an item being as much work whatever its lanes hold
 		// (Q4_S, 2560 columns: three items per pair instead of four; 19456 rows
-		// 17.1 -> 14.6 us with the byte masks of vec_dot). Only Q4_S, whose VALU
-		// work bounds it: Q8_0 was no faster with it (17.3 -> 17.7 us).
+		// 17.4 -> 14.9 us per launch of a graph, with the byte masks of vec_dot).
+		// Only Q4_S, whose VALU work bounds it: Q8_0 was no faster with it (17.3 ->
+		// 17.7 us).
 		template <int F>
 		bool vec_joint(int cols)
 		{
