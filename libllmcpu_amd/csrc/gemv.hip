@@ -1521,12 +1521,20 @@ namespace nnchip
 	// 5.5 / 7.9 and 6.4 / 7.7, 4096 x 384 8.1 / 7.7 and 9.3 / 8.0; Q4_S 640 x 384
 	// 7.3 / 8.1 and 8.4 / 8.4, 2048 x 448 8.2 / 8.3 and 9.6 / 7.9 (replays of a graph,
 	// where the launch is cheap, 6.9 / 4.2 for BF16 640 x 128, 6.5 / 4.6 for Q8_0
-	// 640 x 384). The lines are at numbers of columns, not of rows, so that a
-	// matrix gets the same bits alone and in a group.
-	bool gemv_stages_x(int cols, int n_batch, int format)
+	// 640 x 384). BF16 matrices of 20 000 rows and more (vocabularies) give
+	// gemv_kernel work-groups enough, and up to eight vectors leave it little
+	// besides the weights: eager calls of one stream and of three, 2 and 8
+	// vectors, 151 936 x 1024 60 / 75 and 71 / 79, 50 / 59 and 55 / 61; x 1536 91 /
+	// 111 and 108 / 115, 76 / 94 and 88 / 96; 32 000 x 1024 17.5 / 20.2 and 18.9 /
+	// 20.4 (12 vectors 20.4 / 20.5, 16 22.1 / 20.6); but x 640 52.8 / 49.7 and
+	// 60.7 / 51.6; and where one K split takes all the columns, up to 512, for
+	// any number: 50 000 x 448, 2 and 12 vectors, 22 and 12 % faster. The rows
+	// are one matrix's; see gemv_launch_vectors.
+	bool gemv_stages_x(int rows, int cols, int n_batch, int format)
 	{
 		if (gemv_vec_fits(cols, n_batch, format)) return false;
 		if (n_batch > kGemvMaxBatch) return true;
+		if (format == kGemvBf16 && rows >= 20000) return cols > 512 && cols <= 2048 && (cols < 864 || n_batch > 8);
 		return format == kGemvBf16 ? cols > 256 && cols <= 2048 : cols > 384 && cols <= 6144;
 	}
 

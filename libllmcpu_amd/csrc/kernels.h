@@ -273,9 +273,9 @@ namespace nnchip
 	// K splits of gemv_kernel.
 	void gemv_plan(int cols, int n_batch, int format, int& n_split, int& split_blocks);
 
-	// Whether a call runs with its X staged (gemv_params::xs), and the bytes that
-	// takes.
-	bool gemv_stages_x(int cols, int n_batch, int format);
+	// Whether a launch over a matrix of `rows` rows runs with its X staged
+	// (gemv_params::xs), and the bytes that takes.
+	bool gemv_stages_x(int rows, int cols, int n_batch, int format);
 	size_t gemv_staged_bytes(int cols, int n_batch, int format);
 
 	// Most vectors per launch of a gemv of n_batch.

@@ -1181,12 +1181,13 @@ namespace
 		p.rows = acc;
 	}
 
-	// Scratch of one launch of nb vectors: X staged as matrix operands, or the
-	// K splits' partial sums.
-	static size_t gemv_scratch_bytes(int rows, int cols, int nb, int format)
+	// Scratch of one launch of nb vectors over matrices of `rows` rows in all, the
+	// first of mat_rows: X staged as matrix operands, or the K splits' partial
+	// sums.
+	static size_t gemv_scratch_bytes(int rows, int mat_rows, int cols, int nb, int format)
 	{
 		if (nnchip::gemv_vec_fits(cols, nb, format)) return 0;
-		if (nnchip::gemv_stages_x(cols, nb, format)) return nnchip::gemv_staged_bytes(cols, nb, format);
+		if (nnchip::gemv_stages_x(mat_rows, cols, nb, format)) return nnchip::gemv_staged_bytes(cols, nb, format);
 		int n_split, split_blocks;
 		nnchip::gemv_plan(cols, nb, format, n_split, split_blocks);
 		return n_split > 1 ? static_cast<size_t>(n_split) * nb * static_cast<size_t>(rows) * sizeof(float) : 0;
@@ -1196,12 +1197,13 @@ namespace
 	// captured into a graph and the scratch would have to grow (nothing can be
 	// allocated then), one, on the one-vector kernel. (A rest after the last
 	// whole launch can need more than they do: its K splits' partials.)
-	static uint32_t gemv_chunk(const nnc_hip_kv* kv, int rows, int cols, uint32_t n_batch, int format, uint32_t most)
+	static uint32_t gemv_chunk(const nnc_hip_kv* kv, int rows, int mat_rows, int cols, uint32_t n_batch, int format,
+	                           uint32_t most)
 	{
 		if (n_batch == 1) return 1;
 		size_t need = 0;
 		for (uint32_t nb : {std::min(n_batch, most), n_batch % most})
-			if (nb) need = std::max(need, gemv_scratch_bytes(rows, cols, static_cast<int>(nb), format));
+			if (nb) need = std::max(need, gemv_scratch_bytes(rows, mat_rows, cols, static_cast<int>(nb), format));
 		if (need > kv->gemv_part.bytes && nnchip::gemv_vec_fits(cols, 1, format) && capturing(kv)) return 1;
 		return most;
 	}
@@ -1209,7 +1211,7 @@ namespace
 	// Weight gemvs over the same X on the context's stream: one launch per
 	// chunk of gemv_chunk vectors for all the matrices together (stacked along
 	// the rows), or one per matrix when a matrix other than the last has a row
-	// count that is not a multiple of 16 or their rows ask for different chunks.
+	// count that is not a multiple of 16 or their rows ask for different launches.
 	static nnc_status gemv_impl(nnc_hip_kv* kv, int format, int n_mat, const nnc_hip_gemv_mat* mats, const float* X,
 	                     size_t x_stride, const float* XSUM, size_t xsum_stride, uint32_t cols, uint32_t n_batch)
 	{
@@ -1243,13 +1245,19 @@ namespace
 			return fail(NNC_ERR_INVALID_ARGUMENT, "strides %zu / %zu for %u columns", x_stride, xsum_stride, cols);
 		if ((reinterpret_cast<uintptr_t>(X) & 15) || x_stride % 4 != 0)
 			return fail(NNC_ERR_INVALID_ARGUMENT, "X must be 16-byte aligned, x_stride a multiple of 4");
-		int most = 0;
-		for (int m = 0; m < n_mat; ++m)
+		// The launches' sizes and kernels go by one matrix's rows: those of a group
+		// whose matrices differ in them run by themselves, so that each gets the
+		// bits of its own call.
+		const int ncols = static_cast<int>(cols), mat_rows = static_cast<int>(mats[0].rows);
+		const int n_all = static_cast<int>(std::min<uint32_t>(n_batch, INT_MAX));
+		const int most = nnchip::gemv_launch_vectors(mat_rows, ncols, n_all, format);
+		for (int m = 1; m < n_mat; ++m)
 		{
-			const int v = nnchip::gemv_launch_vectors(static_cast<int>(mats[m].rows), static_cast<int>(cols),
-			                                          static_cast<int>(std::min<uint32_t>(n_batch, INT_MAX)), format);
-			if (m > 0 && v != most) stackable = false;
-			most = v;
+			const int r = static_cast<int>(mats[m].rows);
+			if (nnchip::gemv_launch_vectors(r, ncols, n_all, format) != most) stackable = false;
+			for (int nb : {std::min(n_all, most), n_all % most})
+				if (nb && nnchip::gemv_stages_x(r, ncols, nb, format) != nnchip::gemv_stages_x(mat_rows, ncols, nb, format))
+					stackable = false;
 		}
 		if (!stackable)
 		{
@@ -1260,7 +1268,7 @@ namespace
 		}
 		uint32_t rows[nnchip::kGemvMaxMats];
 		for (int m = 0; m < n_mat; ++m) rows[m] = mats[m].rows;
-		const uint32_t chunk = gemv_chunk(kv, static_cast<int>(total), static_cast<int>(cols), n_batch, format, most);
+		const uint32_t chunk = gemv_chunk(kv, static_cast<int>(total), mat_rows, ncols, n_batch, format, most);
 		for (uint32_t t0 = 0; t0 < n_batch; t0 += chunk)
 		{
 			const int nb = static_cast<int>(std::min<uint32_t>(n_batch - t0, chunk));
@@ -1269,9 +1277,9 @@ namespace
 			stack_rows(p, rows, n_mat);
 			p.n_split = 1;
 			p.split_blocks = static_cast<int>(cols / 32);
-			if (const size_t bytes = gemv_scratch_bytes(p.rows, static_cast<int>(cols), nb, format))
+			if (const size_t bytes = gemv_scratch_bytes(p.rows, mat_rows, ncols, nb, format))
 				if (nnc_status s = reserve(kv, kv->gemv_part, bytes, "gemv scratch")) return s;
-			if (nnchip::gemv_stages_x(static_cast<int>(cols), nb, format))
+			if (nnchip::gemv_stages_x(mat_rows, ncols, nb, format))
 			{
 				p.xs = kv->gemv_part.ptr;
 				p.x_tiles = (nb + 15) / 16;

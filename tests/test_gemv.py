@@ -615,6 +615,37 @@ def test_hip_gemv_q4_s_block_sums_at_the_limit(orc, n):
                 assert np.array_equal(got[n // 2].astype(np.float64), want, equal_nan=True)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [19984, 20011])
+def test_hip_gemv_few_vectors_of_tall_matrices(orc, rows):
+    """Both sides of the line at 20 000 rows of BF16, and of its lines at columns and
+    vectors; a group with a smaller matrix gives each the bits of its own call."""
+    import libllmcpu_amd as nh
+    from libllmcpu_amd import hip_rt
+
+    for cols, n in ((320, 3), (832, 2), (864, 8), (864, 9), (2048, 2)):
+        rng = np.random.default_rng(rows + cols + n)
+        w = orc.bf16_round((rng.standard_normal((rows, cols)) * 0.05).astype(np.float32))
+        x = (rng.standard_normal((n, cols)) * 2).astype(np.float32)
+        print(f"case gemv bf16 {rows} x {cols}, {n} vectors", flush=True)
+        with nh.KVCache([16], [64]) as kv:
+            got = kv.gemv("bf16", (w,), x, rows=rows, cols=cols)
+            assert np.all(np.abs(got.astype(np.float64) - oracle_gemv(orc, "bf16", (w,), x)) <= bound("bf16", (w,), x))
+            few = kv.gemv("bf16", (w[:48],), x, rows=48, cols=cols)
+            dev = [hip_rt.malloc(a.nbytes) for a in (w, x)] + [hip_rt.malloc(n * (48 + rows) * 4)]
+            try:
+                for d, a in zip(dev, (w, x)):
+                    hip_rt.to_device(d, a)
+                kv.gemv_group_device("bf16", [((dev[0],), dev[2], 48), ((dev[0],), dev[2] + 4 * n * 48, rows)], dev[1], cols=cols, n_batch=n)
+                kv.sync()
+                both = hip_rt.to_host(np.empty(n * (48 + rows), np.float32), dev[2])
+                assert np.array_equal(both[:n * 48].reshape(n, 48).view(np.uint32), few.view(np.uint32)), (cols, n)
+                assert np.array_equal(both[n * 48:].reshape(n, rows).view(np.uint32), got.view(np.uint32)), (cols, n)
+            finally:
+                for d in dev:
+                    hip_rt.free(d)
+
+
 # Few rows of many columns: 64 vectors at a time (a rest of 1, 6 and 32), and 16
 # at a time (a rest of 1 and 16).
 FEW_ROWS = [(40, 7168, 65), (129, 9760, 70), (72, 7200, 96), (24, 8800, 17), (33, 9728, 32)]

@@ -127,9 +127,9 @@ def many_vectors_of_few_wide_rows(rt, nh):
             assert launched(fmt, 1024, 2560, 80) == [("gemv_tile_kernel", 80, 1)]
         assert [g[:2] for g in launched("bf16", 640, 9728, 32)] == [("gemv_kernel", 16)] * 2
         for fmt in FORMATS:
-            for cols in (512, 2560, 6144, 9728, 16384):
-                for n in (2, 16, 17, 40, 64, 65, 100, 130, 1030):
-                    for rows in ((4096, 1024, 1024), (1024, 1024), (1040, 3072, 16)):
+            for cols in (512, 1024, 2560, 6144, 9728, 16384):
+                for n in (2, 8, 9, 16, 17, 40, 64, 65, 100, 130, 1030):
+                    for rows in ((4096, 1024, 1024), (1024, 1024), (1040, 3072, 16), (32000, 1024), (16, 32000)):
                         alone = [launched(fmt, r, cols, n) for r in rows]
                         group = launched(fmt, rows, cols, n)
                         want = alone[0] if all(a == alone[0] for a in alone) else [x for a in alone for x in a]
@@ -152,6 +152,23 @@ def narrow_batches_are_one_launch(rt, nh):
                         assert route(got) == [("gemv_kernel", n, 1)] and not got[0]["scratch"], (fmt, cols, n)
                     else:
                         assert [r[0] for r in route(got)] == ["gemv_stage_x_kernel", "gemv_batch_kernel"], (fmt, cols, n)
+
+
+@check
+def few_vectors_of_tall_bf16_matrices(rt, nh):
+    """20 000 rows and more keep gemv_kernel up to eight vectors, and for any number
+    where one K split takes all the columns."""
+    with nh.KVCache([16], [64]) as kv:
+        for rows in (19984, 20000, 151936):
+            for cols, n in ((320, 16), (512, 2), (544, 2), (640, 8), (832, 2), (864, 2), (1024, 8), (1024, 9), (2048, 2), (2048, 16)):
+                rt.clear()
+                gemv(kv, "bf16", n, rows, cols)
+                kernel = [r[0] for r in route(rt.launches()) if "stage_x" not in r[0]][0]
+                split = rows >= 20000 and (cols <= 512 or (cols >= 864 and n <= 8))
+                assert kernel == ("gemv_kernel" if split else "gemv_batch_kernel"), (rows, cols, n, kernel)
+            rt.clear()
+            gemv(kv, "q8_0", 2, rows, 1024)
+            assert route(rt.launches())[-1][0] == "gemv_batch_kernel"
 
 
 @check
