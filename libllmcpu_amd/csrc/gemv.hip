@@ -1521,20 +1521,29 @@ namespace nnchip
 	// 5.5 / 7.9 and 6.4 / 7.7, 4096 x 384 8.1 / 7.7 and 9.3 / 8.0; Q4_S 640 x 384
 	// 7.3 / 8.1 and 8.4 / 8.4, 2048 x 448 8.2 / 8.3 and 9.6 / 7.9 (replays of a graph,
 	// where the launch is cheap, 6.9 / 4.2 for BF16 640 x 128, 6.5 / 4.6 for Q8_0
-	// 640 x 384). BF16 matrices of 20 000 rows and more (vocabularies) give
-	// gemv_kernel work-groups enough, and up to eight vectors leave it little
-	// besides the weights: eager calls of one stream and of three, 2 and 8
-	// vectors, 151 936 x 1024 60 / 75 and 71 / 79, 50 / 59 and 55 / 61; x 1536 91 /
-	// 111 and 108 / 115, 76 / 94 and 88 / 96; 32 000 x 1024 17.5 / 20.2 and 18.9 /
-	// 20.4 (12 vectors 20.4 / 20.5, 16 22.1 / 20.6); but x 640 52.8 / 49.7 and
-	// 60.7 / 51.6; and where one K split takes all the columns, up to 512, for
-	// any number: 50 000 x 448, 2 and 12 vectors, 22 and 12 % faster. The rows
-	// are one matrix's; see gemv_launch_vectors.
+	// 640 x 384). BF16 matrices of many rows give gemv_kernel work-groups enough,
+	// and up to eight vectors leave it little besides the weights: eager calls of
+	// one stream and of three, 2 and 8 vectors, 151 936 x 1024 60 / 75 and 71 / 79,
+	// 50 / 59 and 55 / 61; x 1536 91 / 111 and 108 / 115, 76 / 94 and 88 / 96;
+	// 32 000 x 1024 17.5 / 20.2 and 18.9 / 20.4 (12 vectors 20.4 / 20.5, 16 22.1 /
+	// 20.6); but x 640 52.8 / 49.7 and 60.7 / 51.6; and where one K split takes
+	// all the columns, up to 512, for any number: 50 000 x 448, 2 and 12 vectors,
+	// 22 and 12 % faster. Of fewer rows, two matrices in a group (gate and up) of
+	// 8704 to 10 752 rows leave gemv_batch_kernel a short last round (9216 x 1280,
+	// x 1440, x 1536, 2 vectors: 16 to 21 % faster in gemv_kernel, 8 vectors 12 to
+	// 18; 11 264 x 1280 5 % slower), and from 1664 columns on so do most (6144 x
+	// 1792 11 %, 8192 x 2048 2 and with three streams 12 %). The rows are one
+	// matrix's; see gemv_launch_vectors.
 	bool gemv_stages_x(int rows, int cols, int n_batch, int format)
 	{
 		if (gemv_vec_fits(cols, n_batch, format)) return false;
 		if (n_batch > kGemvMaxBatch) return true;
-		if (format == kGemvBf16 && rows >= 20000) return cols > 512 && cols <= 2048 && (cols < 864 || n_batch > 8);
+		if (format == kGemvBf16 && rows >= 20000 && cols <= 512) return false;
+		if (format == kGemvBf16 && n_batch <= 8 && rows >= 6144)
+		{
+			const int most = rows >= 20000 ? 863 : (rows >= 8704 && rows <= 10752 ? 1151 : 1663);
+			return cols > 256 && cols <= most;
+		}
 		return format == kGemvBf16 ? cols > 256 && cols <= 2048 : cols > 384 && cols <= 6144;
 	}
 

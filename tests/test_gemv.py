@@ -616,14 +616,14 @@ def test_hip_gemv_q4_s_block_sums_at_the_limit(orc, n):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows", [19984, 20011])
+@pytest.mark.parametrize("rows", [6143, 8704, 19984, 20011])
 def test_hip_gemv_few_vectors_of_tall_matrices(orc, rows):
-    """Both sides of the line at 20 000 rows of BF16, and of its lines at columns and
+    """Both sides of the lines at rows of BF16, and of their lines at columns and
     vectors; a group with a smaller matrix gives each the bits of its own call."""
     import libllmcpu_amd as nh
     from libllmcpu_amd import hip_rt
 
-    for cols, n in ((320, 3), (832, 2), (864, 8), (864, 9), (2048, 2)):
+    for cols, n in ((320, 3), (832, 2), (864, 8), (864, 9), (1152, 2), (1664, 8), (2048, 2)):
         rng = np.random.default_rng(rows + cols + n)
         w = orc.bf16_round((rng.standard_normal((rows, cols)) * 0.05).astype(np.float32))
         x = (rng.standard_normal((n, cols)) * 2).astype(np.float32)

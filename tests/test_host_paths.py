@@ -156,18 +156,20 @@ def narrow_batches_are_one_launch(rt, nh):
 
 @check
 def few_vectors_of_tall_bf16_matrices(rt, nh):
-    """20 000 rows and more keep gemv_kernel up to eight vectors, and for any number
-    where one K split takes all the columns."""
+    """Matrices of many rows keep gemv_kernel up to eight vectors from a number of
+    columns on, and 20 000 rows for any number where one K split takes them all."""
     with nh.KVCache([16], [64]) as kv:
-        for rows in (19984, 20000, 151936):
-            for cols, n in ((320, 16), (512, 2), (544, 2), (640, 8), (832, 2), (864, 2), (1024, 8), (1024, 9), (2048, 2), (2048, 16)):
-                rt.clear()
-                gemv(kv, "bf16", n, rows, cols)
-                kernel = [r[0] for r in route(rt.launches()) if "stage_x" not in r[0]][0]
-                split = rows >= 20000 and (cols <= 512 or (cols >= 864 and n <= 8))
-                assert kernel == ("gemv_kernel" if split else "gemv_batch_kernel"), (rows, cols, n, kernel)
+        for rows, from_cols in ((6143, 2080), (6144, 1664), (8703, 1664), (8704, 1152), (10752, 1152), (10753, 1664),
+                                (19999, 1664), (20000, 864), (151936, 864)):
+            for cols in (320, 512, 544, 640, 832, 864, 1120, 1152, 1632, 1664, 2048, 2080):
+                for n in (2, 8, 9, 16):
+                    rt.clear()
+                    gemv(kv, "bf16", n, rows, cols)
+                    kernel = [r[0] for r in route(rt.launches()) if "stage_x" not in r[0]][0]
+                    split = cols > 2048 or rows >= 20000 and cols <= 512 or n <= 8 and cols >= from_cols
+                    assert kernel == ("gemv_kernel" if split else "gemv_batch_kernel"), (rows, cols, n, kernel)
             rt.clear()
-            gemv(kv, "q8_0", 2, rows, 1024)
+            gemv(kv, "q8_0", 2, rows, 1664)
             assert route(rt.launches())[-1][0] == "gemv_batch_kernel"
 
 
