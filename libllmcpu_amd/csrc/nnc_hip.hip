@@ -1250,8 +1250,8 @@ namespace
 		// bits of its own call.
 		const int ncols = static_cast<int>(cols), mat_rows = static_cast<int>(mats[0].rows);
 		const int n_all = static_cast<int>(std::min<uint32_t>(n_batch, INT_MAX));
-		const int most = nnchip::gemv_launch_vectors(mat_rows, ncols, n_all, format);
-		for (int m = 1; m < n_mat; ++m)
+		const int most = n_all > 1 ? nnchip::gemv_launch_vectors(mat_rows, ncols, n_all, format) : nnchip::kGemvWideBatch;
+		for (int m = 1; m < n_mat && n_all > 1; ++m) // (one vector: one kernel for all rows)
 		{
 			const int r = static_cast<int>(mats[m].rows);
 			if (nnchip::gemv_launch_vectors(r, ncols, n_all, format) != most) stackable = false;
